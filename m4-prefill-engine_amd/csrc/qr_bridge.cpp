@@ -310,9 +310,9 @@ int launch_ws(const qr::GemmParams& p0, float* fixed_ws, size_t fixed_floats) {
         }
         return 0;
     }
-    p.ksplit = qr::gemm_pick_ksplit(p);
+    qr::gemm_plan(p);
     if (p.ksplit > 1) {
-        if (int rc = workspace(qr::gemm_workspace_floats(p, p.ksplit), &p.ws)) return rc;
+        if (int rc = workspace(qr::gemm_workspace_floats(p), &p.ws)) return rc;
     }
     hipError_t e = qr::launch_gemm(p, g_stream);
     if (e != hipSuccess) {
@@ -712,8 +712,8 @@ int m4_bridge_prefill_layer_ex_kv(void* X, void* w_attn, void* Wq, void* Wk, voi
         g.ngroups = 3;
         g.Wx[0] = static_cast<const uint8_t*>(Wk); g.Yx[0] = k; g.Nx[0] = HK;
         g.Wx[1] = static_cast<const uint8_t*>(Wv); g.Yx[1] = v; g.Nx[1] = HK;
+        qr::gemm_plan(g);
         if (qr::gemm_grouped_ok(g)) {
-            g.ksplit = 1;
             rc = check(qr::launch_gemm(g, g_stream), "layer qkv");
         } else {
             rc = proj(a, Wq, nullptr, q, nullptr, HQ, dm, D);

@@ -122,21 +122,6 @@ struct Cfg {
 // take the even or the odd values) hit distinct bank groups.
 __device__ __forceinline__ uint32_t xswz(uint32_t r) { return (r ^ (r >> 3)) & 7u; }
 
-__device__ __forceinline__ void tile_of(uint32_t bid, uint32_t nt_m, uint32_t nt_n, uint32_t gm_req, uint32_t& tm,
-                                        uint32_t& tn) {
-    const uint32_t T = nt_m * nt_n;
-    uint32_t t = bid;
-    if (T % 8 == 0) t = (bid % 8) * (T / 8) + bid / 8;
-    const uint32_t GM = gm_req ? gm_req : 2;
-    const uint32_t per_group = GM * nt_n;
-    const uint32_t grp = t / per_group;
-    const uint32_t first = grp * GM;
-    const uint32_t gm = min(GM, nt_m - first);
-    const uint32_t in = t % per_group;
-    tm = first + in % gm;
-    tn = in / gm;
-}
-
 }  // namespace rb
 
 // SPLIT: the instance writes split-K partials (the stores are compiled only
@@ -196,7 +181,7 @@ gemm_rb_kernel(GemmParams p) {
     const uint32_t M = p.M, N = p.N, K = p.K;
     const uint32_t nt_m = (M + C::BM - 1) / C::BM, nt_n = (N + C::BN - 1) / C::BN;
     uint32_t tmi, tni;
-    rb::tile_of(bid, nt_m, nt_n, p.group_m, tmi, tni);
+    tile_of(bid, nt_m, nt_n, p.group_m, tmi, tni);
     const int m0 = tmi * C::BM, n0 = tni * C::BN;
     const uint32_t ksplit = p.ksplit ? p.ksplit : 1;
     const uint32_t kz = blockIdx.y;
@@ -685,7 +670,7 @@ static hipError_t rb_launch_cfg(const GemmParams& p, hipStream_t st) {
     using C = rb::Cfg<TM, TN, NW, WR, KG, DUAL, rb::use_stager(F, TN, NW, KG, DUAL)>;
     auto kern = gemm_rb_kernel<F, TM, TN, NW, WR, KG, DUAL, kWeightStages, false>;
     if constexpr (KG > 1) {
-        if (p.ksplit > 1 || p.K % (64 * KG) != 0) return hipErrorInvalidValue;  // rb_pick never asks for these
+        if (p.ksplit > 1 || p.K % (64 * KG) != 0) return hipErrorInvalidValue;  // gemm_plan never asks for these
     } else {
         if (p.ksplit > 1) kern = gemm_rb_kernel<F, TM, TN, NW, WR, KG, DUAL, kWeightStages, true>;
     }
@@ -708,9 +693,9 @@ static hipError_t rb_launch_fmt(const GemmParams& p, hipStream_t st) {
     if constexpr (DUAL) {
         return rb_launch_cfg<F, QR_RB_DUAL, true>(p, st);
     } else if constexpr (F == QUANT_VAR_RATE_AFFINE || F == QUANT_EXL3) {
-        return rb_launch_cfg<F, QR_RB_MID, false>(p, st);  // rb_pick's only shape for these formats
+        return rb_launch_cfg<F, QR_RB_MID, false>(p, st);  // the only shape for these formats
     } else {
-        switch (rb_pick(F, p.M, p.N, p.K, false)) {
+        switch (p.shape) {
             case 0: return rb_launch_cfg<F, QR_RB_BIG, false>(p, st);
             case 3: return rb_launch_cfg<F, QR_RB_BIG_K, false>(p, st);
             case 4: return rb_launch_cfg<F, QR_RB_MID64, false>(p, st);
@@ -723,6 +708,8 @@ static hipError_t rb_launch_fmt(const GemmParams& p, hipStream_t st) {
 
 template <int F>
 hipError_t launch_gemm_format(const GemmParams& p, hipStream_t st) {
+    if constexpr (wide_format(F))
+        if (p.shape == 7 || p.shape == 8) return launch_gemm_wide_format<F>(p, st);
     return p.W2 ? rb_launch_fmt<F, true>(p, st) : rb_launch_fmt<F, false>(p, st);
 }
 

@@ -113,9 +113,7 @@ static hipError_t launch_gemm_main(const GemmParams& p, hipStream_t st) {
     }
 }
 
-hipError_t launch_gemm(const GemmParams& p0, hipStream_t st) {
-    GemmParams p = p0;
-    p.group_m = gemm_group_m(p);
+hipError_t launch_gemm(const GemmParams& p, hipStream_t st) {
     hipError_t e = launch_gemm_main(p, st);
     if (e == hipSuccess && p.ksplit > 1)
         e = launch_splitk_reduce(p.ws, p.ksplit, p.M, p.N, p.W2 != nullptr, p.R, p.Y, p.head_D, st);
@@ -130,35 +128,79 @@ static uint32_t tiles_of(const GemmParams& p, const RbShape& d) {
 }
 
 bool gemm_grouped_ok(const GemmParams& p) {
-    if (p.ngroups < 2 || p.ngroups > 3 || p.W2 || p.R) return false;
-    // every group must take the shape group 0 takes, and the grid needs no K split
-    const int s0 = rb_pick(p.format, p.M, p.N, p.K, false);
-    for (uint32_t g = 1; g < p.ngroups; g++)
-        if (rb_pick(p.format, p.M, p.Nx[g - 1], p.K, false) != s0) return false;
-    return gemm_pick_ksplit(p) == 1;
+    // the groups share the shape; the grid needs no K split
+    return p.ngroups >= 2 && p.ngroups <= 3 && !p.W2 && !p.R && p.ksplit <= 1;
 }
 
-uint32_t gemm_pick_ksplit(const GemmParams& p) {
-    const int shape = rb_pick(p.format, p.M, p.N, p.K, p.W2 != nullptr);
-    if (shape == 5 || shape == 6) return 1;  // K groups: the tile takes the whole K range
-    const RbShape d = rb_dims(shape);
-    const uint32_t T = tiles_of(p, d);
-    // One workgroup fits a CU (its registers), so the grid runs in waves of
-    // 256 workgroups: split K (powers of two, whole 256-element super-blocks,
-    // >= 512 of K per split) while the grid still fits one such wave.
-    uint32_t ks = 1;
-    while (T * ks * 2 <= 256 && p.K % (256 * ks * 2) == 0 && p.K / (ks * 2) >= 512) ks *= 2;
-    return ks;
+// One workgroup fits a CU, so a grid runs in waves of 256 tiles.  What a wave
+// takes, in us at K = 4096 (it is proportional to K but for ~5 us), per shape:
+// `lo` while at most half of the CUs have a tile, rising to `hi` when all have
+// (the clock falls as the chip fills).  Measured on MLX and Q4_0 weights (they
+// agree to 5%; ternary is ~10% faster at every shape) and on Q4_K, whose decode
+// is the heaviest; e.g. MLX at N = 14336: M = 900 128 x 128 tiles 142.7,
+// 128 x 256 121.2, 256 x 256 107.4; M = 450 71.4 / 61.6 / 82.4; M = 256
+// 37.0 / 52.5 / 81.5.
+struct WaveCost {
+    float lo, hi;
+};
+static WaveCost wave_cost(int shape, bool q4k) {
+    switch (shape) {
+        case 0: return q4k ? WaveCost{68, 77} : WaveCost{51, 72};
+        case 3: return q4k ? WaveCost{61, 77} : WaveCost{50, 72};
+        case 1: return q4k ? WaveCost{39.5f, 47} : WaveCost{31, 39};
+        case 4: return q4k ? WaveCost{33, 36} : WaveCost{25, 32};
+        case 5: return q4k ? WaveCost{24, 29} : WaveCost{19, 26};
+        case 6: return q4k ? WaveCost{27, 31} : WaveCost{18.5f, 25};
+        case 7: return q4k ? WaveCost{97, 130} : WaveCost{81, 122};
+        case 8: return q4k ? WaveCost{94, 130} : WaveCost{79, 122};
+        default: return q4k ? WaveCost{66, 82} : WaveCost{53, 72};  // 2: SwiGLU 128 x 128
+    }
+}
+static float plan_cost(const GemmParams& p, int shape, uint32_t ks) {
+    const WaveCost w = wave_cost(shape, p.format == QUANT_Q4_K);
+    const uint32_t T = tiles_of(p, rb_dims(shape)) * ks, rem = T % 256;
+    float c = (float)(T / 256) * w.hi;
+    if (rem) c += w.lo + (rem > 128 ? (w.hi - w.lo) * (float)(rem - 128) / 128.0f : 0.0f);
+    c *= (float)p.K / (4096.0f * (float)ks);
+    // the partials' round trip (~4.5 TB/s) and the reduction kernel
+    if (ks > 1) c += 4.0f + (float)ks * (float)p.M * (float)p.N * (p.W2 ? 16.0f : 8.0f) / 4.5e6f;
+    return c;
 }
 
-size_t gemm_workspace_floats(const GemmParams& p, uint32_t ks) {
-    return ks > 1 ? (size_t)ks * p.M * p.N * (p.W2 != nullptr ? 2 : 1) : 0;
+// The base shape with its K split, unless another shape without a split is
+// cheaper by its tile counts (so no call needs split-K partials that the base
+// choice would not).
+void gemm_plan(GemmParams& p) {
+    const bool dual = p.W2 != nullptr;
+    p.shape = rb_pick(p.format, p.M, p.N, p.K, dual);
+    p.ksplit = 1;
+    if (p.shape != 5 && p.shape != 6) {  // K groups: the tile takes the whole K range
+        // split K (powers of two, whole 256-element super-blocks, >= 512 of K
+        // per split) while the grid still fits one wave
+        const uint32_t T = tiles_of(p, rb_dims(p.shape));
+        while (T * p.ksplit * 2 <= 256 && p.K % (256 * p.ksplit * 2) == 0 && p.K / (p.ksplit * 2) >= 512) p.ksplit *= 2;
+    }
+    if (p.format != QUANT_VAR_RATE_AFFINE && p.format != QUANT_EXL3) {  // those have one shape
+        const bool heavy = p.format == QUANT_Q4_K || p.format == QUANT_TERNARY_1_58;
+        const bool groups_ok = p.K % 128 == 0, wide = groups_ok && wide_format(p.format);
+        const int cand[6] = {dual ? 2 : 1, dual ? -1 : (heavy ? 3 : 0), dual ? (wide ? 8 : -1) : (wide ? 7 : -1),
+                             dual || !groups_ok ? -1 : 6, dual || !groups_ok || p.M > 128 ? -1 : 5, dual ? -1 : 4};
+        float best = 0.97f * plan_cost(p, p.shape, p.ksplit);
+        for (int s : cand) {
+            if (s < 0) continue;
+            const float c = plan_cost(p, s, 1);
+            if (c < best) {
+                best = c;
+                p.shape = s;
+                p.ksplit = 1;
+            }
+        }
+    }
+    p.group_m = (p.M + rb_dims(p.shape).bm - 1) / rb_dims(p.shape).bm >= 4 ? 4u : 2u;
 }
 
-uint32_t gemm_group_m(const GemmParams& p) {
-    const RbShape d = rb_dims(rb_pick(p.format, p.M, p.N, p.K, p.W2 != nullptr));
-    const uint32_t nt_m = (p.M + d.bm - 1) / d.bm;
-    return nt_m >= 4 ? 4u : 2u;
+size_t gemm_workspace_floats(const GemmParams& p) {
+    return p.ksplit > 1 ? (size_t)p.ksplit * p.M * p.N * (p.W2 != nullptr ? 2 : 1) : 0;
 }
 
 }  // namespace qr

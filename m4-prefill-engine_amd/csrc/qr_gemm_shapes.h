@@ -21,7 +21,8 @@ namespace qr {
 //   5 (M <= 128, wide N): QR_RB_KG (4, 1, 4, 1, 2 -> 128 x 64: two K groups
 //                  of two column waves take alternate K steps and meet in LDS,
 //                  so 224 workgroups cover M = 128, N = 14336 with no K split)
-//   dual (SwiGLU): 4, 1, 4 -> 128 x 128 outputs (gate + up: 256 weight columns)
+//   2 (SwiGLU): 4, 1, 4 -> 128 x 128 outputs (gate + up: 256 weight columns)
+//   7, 8 (SwiGLU): 256 x 256, 256 x 128 outputs (qr_gemm_wide.hip)
 #define QR_RB_BIG 4, 2, 4, 1, 1
 #define QR_RB_BIG_K 4, 1, 8, 1, 1
 #define QR_RB_MID 4, 1, 4, 1, 1
@@ -35,7 +36,11 @@ template <int TM, int TN, int NW, int WR, int KG> struct ShapeOf {
 struct RbShape {
     uint32_t bm, bn;
 };
-// Shape choice.  At M >= 1024 the wide tile is used while it alone fills the
+// Formats with the 256 x 256 tiles of qr_gemm_wide.hip.
+constexpr bool wide_format(int f) {
+    return f == QUANT_Q4_0 || f == QUANT_MLX_4BIT || f == QUANT_Q4_K || f == QUANT_TERNARY_1_58 || f == QUANT_MLX_4BIT_G64;
+}
+// Base shape choice (gemm_plan compares it with the others by tile count).  At M >= 1024 the wide tile is used while it alone fills the
 // 256 CUs; when it cannot (N small), 128 x 128 tiles give twice the tiles, so
 // the K split -- whose fp32 partials are M x N x 4 bytes written and read per
 // extra split -- is halved or avoided.
@@ -78,9 +83,29 @@ inline RbShape rb_dims(int s) {
         case 1: return {ShapeOf<QR_RB_MID>::bm, ShapeOf<QR_RB_MID>::bn};
         case 4: return {ShapeOf<QR_RB_MID64>::bm, ShapeOf<QR_RB_MID64>::bn};
         case 5: return {ShapeOf<QR_RB_KG>::bm, ShapeOf<QR_RB_KG>::bn};
+        case 7: return {256, 256};
+        case 8: return {256, 128};
         case 6: return {ShapeOf<QR_RB_MID64_KG>::bm, ShapeOf<QR_RB_MID64_KG>::bn};
         default: return {ShapeOf<QR_RB_DUAL>::bm, ShapeOf<QR_RB_DUAL>::bn};
     }
+}
+
+// Workgroup id -> tile (tm, tn) of an nt_m x nt_n grid.  Consecutive ids land
+// on different XCDs: each XCD gets a contiguous run of tiles, grouped gm_req
+// row tiles x many column tiles.
+__device__ __forceinline__ void tile_of(uint32_t bid, uint32_t nt_m, uint32_t nt_n, uint32_t gm_req, uint32_t& tm,
+                                        uint32_t& tn) {
+    const uint32_t T = nt_m * nt_n;
+    uint32_t t = bid;
+    if (T % 8 == 0) t = (bid % 8) * (T / 8) + bid / 8;
+    const uint32_t GM = gm_req ? gm_req : 2;
+    const uint32_t per_group = GM * nt_n;
+    const uint32_t grp = t / per_group;
+    const uint32_t first = grp * GM;
+    const uint32_t gm = min(GM, nt_m - first);
+    const uint32_t in = t % per_group;
+    tm = first + in % gm;
+    tn = in / gm;
 }
 
 // Launches the tiled kernel of format F (plain, or the SwiGLU dual variant when
@@ -88,5 +113,8 @@ inline RbShape rb_dims(int s) {
 // compilation unit (qr_gemm.hip built with -DQR_GEMM_FORMAT=F).
 template <int F>
 hipError_t launch_gemm_format(const GemmParams& p, hipStream_t st);
+// The same for the 256 x 256 tiles of qr_gemm_wide.hip.
+template <int F>
+hipError_t launch_gemm_wide_format(const GemmParams& p, hipStream_t st);
 
 }  // namespace qr

@@ -21,7 +21,8 @@ struct GemmParams {
     // launch_gemm follows the projection with the reduction kernel.
     uint32_t ksplit;
     float* ws;
-    uint32_t group_m;     // row-tiles per XCD tile group (0: kernel default)
+    int shape;            // tile shape (gemm_plan)
+    uint32_t group_m;     // row-tiles per XCD tile group (0: kernel default; gemm_plan)
     // Grouped launch: up to two more projections of the same X (same K,
     // format, head_D; no residual, no SwiGLU, no K split) in the same grid,
     // group g >= 1 writing Yx[g - 1] [M, Nx[g - 1]] from Wx[g - 1].
@@ -31,12 +32,12 @@ struct GemmParams {
     uint32_t Nx[2];
 };
 
+// Tile shape, K split and tile order of p (before launch_gemm).
+void gemm_plan(GemmParams& p);
 hipError_t launch_gemm(const GemmParams& p, hipStream_t st);
-uint32_t gemm_group_m(const GemmParams& p);
-uint32_t gemm_pick_ksplit(const GemmParams& p);
-// Whether launch_gemm can run p's groups (ngroups >= 2) as one grid.
+// Whether launch_gemm can run p's groups (ngroups >= 2) as one grid, as planned.
 bool gemm_grouped_ok(const GemmParams& p);
-size_t gemm_workspace_floats(const GemmParams& p, uint32_t ksplit);
+size_t gemm_workspace_floats(const GemmParams& p);
 // Sums split-K partials ws [ks][dual ? 2 : 1][M][N] in split order and writes
 // the projection epilogue (SwiGLU when dual, + R, fp16, head-major when
 // head_D) -- the second kernel of every split-K projection.

@@ -380,6 +380,50 @@ def test_gemm_decode_bit_exact_mixed_exact_paths(bridge, oracle, fmt, M, K, N):
 
 
 @pytest.mark.parametrize("fmt", [0, 1, 2, 3, 8])
+@pytest.mark.parametrize("layout,M,K,N", [("plain", 500, 128, 22038), ("plain", 513, 256, 22040), ("head", 500, 384, 22016),
+                                          ("residual", 511, 640, 22016), ("swiglu", 500, 128, 9000),
+                                          ("swiglu", 512, 384, 9002)])
+def test_wide_tiles(bridge, oracle, fmt, layout, M, K, N):
+    """The 256 x 256 tiles (more than one wave of 128 x 256 tiles): ragged M
+    and N (an N that is no multiple of 8, whose stores are per element), K of
+    one round of 4 steps (128), two, three and five (the rings of three X
+    pairs and two weight slots wrap at every phase), each output layout and
+    SwiGLU, against the oracle on a row sample with every column."""
+    K = 256 * -(-K // 256) if fmt == 2 else K  # Q4_K: whole super-blocks
+    X = synth.activations(M, K, 170 + fmt, std=0.35)
+    W = weights("quantized", fmt, N, K, 171 + fmt)
+    rows = np.unique(np.r_[0, 1, 31, 32, 127, 128, 255, 256, M - 1])
+    Xs = np.ascontiguousarray(X[rows])
+    Y = empty16(M, N)
+    if layout == "swiglu":
+        Wu = weights("quantized", fmt, N, K, 172 + fmt)
+        bridge.dispatch_swiglu(dev(X), dev(W), dev(Wu), Y, fmt, M, N, K)
+        gold = oracle.swiglu(fmt, Xs, W, Wu, N)
+    elif layout == "head":
+        bridge.dispatch_head_gemm(dev(X), dev(W), Y, fmt, M, N // 64, 64, K)
+        gold = oracle.gemm(fmt, Xs, W, N)
+    elif layout == "residual":
+        R = synth.activations(M, N, 173)
+        bridge.dispatch_gemm_residual(dev(X), dev(W), dev(R), Y, fmt, M, K, N)
+        gold = oracle.gemm(fmt, Xs, W, N, R=np.ascontiguousarray(R[rows]))
+    else:
+        bridge.dispatch_router_gemm(dev(X), dev(W), Y, fmt, M, K, N)
+        gold = oracle.gemm(fmt, Xs, W, N)
+    bridge.synchronize()
+    y = host(Y)
+    if layout == "head":
+        y = y.reshape(N // 64, M, 64).transpose(1, 0, 2).reshape(M, N)
+    tolerance.check_ref(y[rows], gold, what=f"wide {layout} fmt {fmt} {M}x{K}x{N}")
+
+
+@pytest.mark.parametrize("fmt", [0, 2])
+def test_wide_tiles_decode_bit_exact_mixed_exact_paths(bridge, oracle, fmt):
+    """One-hot X through the 256 x 256 tiles with a third of the blocks outside
+    the fast decode's range: every output is one exact product."""
+    test_gemm_decode_bit_exact_mixed_exact_paths(bridge, oracle, fmt, 512, 512, 22016)
+
+
+@pytest.mark.parametrize("fmt", [0, 1, 2, 3, 8])
 @pytest.mark.parametrize("M,K,N", [(1, 4096, 4096), (33, 4096, 4104), (64, 2048, 4096), (17, 1024, 4096)])
 def test_gemm_small_m_wide(bridge, oracle, fmt, M, K, N):
     """The small-M projection (M <= 64) on wide outputs, every format it
