@@ -299,6 +299,14 @@ int launch_ws(const qr::GemmParams& p0, float* fixed_ws, size_t fixed_floats) {
         *ws = g_sk_ws;
         return 0;
     };
+    if (qr::gemv_fits(p)) {
+        hipError_t e = qr::launch_gemv(p, g_stream);
+        if (e != hipSuccess) {
+            set_error("launch_gemv", e);
+            return -6;
+        }
+        return 0;
+    }
     if (qr::skinny_supported(p)) {
         const size_t floats = qr::skinny_workspace_floats(p.M, p.N, p.K);
         float* ws = nullptr;

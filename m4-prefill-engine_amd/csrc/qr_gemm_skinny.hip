@@ -719,6 +719,8 @@ bool skinny_supported(const GemmParams& p) {
     return st_plan(p.format, p.M, p.N, p.K) || sk_plan(p.format, p.M, p.N, p.K, &ks, &gpw);
 }
 
+bool skinny_one_kernel(const GemmParams& p) { return st_plan(p.format, p.M, p.N, p.K); }
+
 hipError_t launch_gemm_skinny(const GemmParams& p, float* ws, hipStream_t st) {
     switch (p.format) {
         case QUANT_Q4_0: return launch_sk_m<QUANT_Q4_0>(p, ws, st);

@@ -44,10 +44,17 @@ size_t gemm_workspace_floats(const GemmParams& p);
 hipError_t launch_splitk_reduce(const float* ws, uint32_t ks, uint32_t M, uint32_t N, bool dual, const _Float16* R,
                                 _Float16* Y, uint32_t head_D, hipStream_t st);
 
+// One-kernel projection or SwiGLU for M <= 16 (no workspace), and whether it
+// takes p.
+bool gemv_fits(const GemmParams& p);
+hipError_t launch_gemv(const GemmParams& p, hipStream_t st);
+
 // Small-M weight-streaming projection (M <= 64, no SwiGLU).  `ws` holds
 // skinny_workspace_floats() floats of split-K partials [split][M][N], summed
 // by launch_splitk_reduce.  Calls that share ws must be ordered on one stream.
 bool skinny_supported(const GemmParams& p);
+// Whether launch_gemm_skinny runs p as one kernel, without a K split.
+bool skinny_one_kernel(const GemmParams& p);
 size_t skinny_workspace_floats(uint32_t M, uint32_t N, uint32_t K);
 hipError_t launch_gemm_skinny(const GemmParams& p, float* ws, hipStream_t st);
 hipError_t launch_dequant(int format, const uint8_t* W, _Float16* out, uint32_t K, uint32_t N, size_t col_bytes,

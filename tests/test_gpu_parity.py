@@ -416,6 +416,43 @@ def test_wide_tiles(bridge, oracle, fmt, layout, M, K, N):
     tolerance.check_ref(y[rows], gold, what=f"wide {layout} fmt {fmt} {M}x{K}x{N}")
 
 
+@pytest.mark.parametrize("fmt", [0, 1, 2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("layout,M,K,N", [("plain", 1, 256, 40), ("plain", 2, 2304, 1000), ("head", 8, 2048, 512),
+                                          ("residual", 16, 512, 2046), ("plain", 1, 512, 14344),
+                                          ("swiglu", 1, 2304, 1000), ("swiglu", 16, 512, 36)])
+def test_few_rows(bridge, oracle, fmt, layout, M, K, N):
+    """The one-kernel projection for up to 16 rows: K of one chunk (seven of
+    the eight waves idle), two and nine (waves with one and two), ragged N, two
+    column tiles per workgroup (N = 14344: an odd tile count's last half
+    empty), every layout and SwiGLU, every format, on every element."""
+    X = synth.activations(M, K, 180 + fmt, std=0.35)
+    kind = "random" if fmt > 3 and fmt != 8 else "quantized"
+    W = weights(kind, fmt, N, K, 181 + fmt)
+    Y = empty16(M, N)
+    if layout == "swiglu":
+        Wu = weights(kind, fmt, N, K, 182 + fmt)
+        bridge.dispatch_swiglu(dev(X), dev(W), dev(Wu), Y, fmt, M, N, K)
+        bridge.synchronize()
+        gold = oracle.swiglu(fmt, X, W, Wu, N)
+        Xd = X.astype(np.float64)
+        Wd, Wud = oracle.dequantize_f64(fmt, W, K, N), oracle.dequantize_f64(fmt, Wu, K, N)
+        tolerance.check(host(Y), gold, tolerance.swiglu_bound(gold, Xd @ Wd.T, Xd @ Wud.T, np.abs(Xd) @ np.abs(Wd).T,
+                                                              np.abs(Xd) @ np.abs(Wud).T, K))
+        return
+    if layout == "head":
+        bridge.dispatch_head_gemm(dev(X), dev(W), Y, fmt, M, N // 64, 64, K)
+        gold = oracle.gemm(fmt, X, W, N, head_D=64).reshape(M, N)
+    elif layout == "residual":
+        R = synth.activations(M, N, 183)
+        bridge.dispatch_gemm_residual(dev(X), dev(W), dev(R), Y, fmt, M, K, N)
+        gold = oracle.gemm(fmt, X, W, N, R=R)
+    else:
+        bridge.dispatch_router_gemm(dev(X), dev(W), Y, fmt, M, K, N)
+        gold = oracle.gemm(fmt, X, W, N)
+    bridge.synchronize()
+    tolerance.check(host(Y), gold, tolerance.gemm_bound(gold, absxw(oracle, fmt, X, W, K, N), K))
+
+
 @pytest.mark.parametrize("fmt", [0, 2])
 def test_wide_tiles_decode_bit_exact_mixed_exact_paths(bridge, oracle, fmt):
     """One-hot X through the 256 x 256 tiles with a third of the blocks outside
