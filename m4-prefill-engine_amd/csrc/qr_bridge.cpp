@@ -307,7 +307,7 @@ int launch_ws(const qr::GemmParams& p0, float* fixed_ws, size_t fixed_floats) {
         }
         return 0;
     }
-    if (qr::skinny_supported(p)) {
+    if (p.ngroups <= 1 && qr::skinny_supported(p)) {
         const size_t floats = qr::skinny_workspace_floats(p.M, p.N, p.K);
         float* ws = nullptr;
         if (int rc = workspace(floats ? floats : 1, &ws)) return rc;
@@ -707,7 +707,7 @@ int m4_bridge_prefill_layer_ex_kv(void* X, void* w_attn, void* Wq, void* Wk, voi
                                       eps, norm_type, g_stream), "layer rmsnorm");
         a = xn;
     }
-    // Q, K, V: one grouped launch when the three fit one grid, else three
+    // Q, K, V: one grouped launch
     if (!rc) {
         qr::GemmParams g{};
         g.format = format;
@@ -720,18 +720,10 @@ int m4_bridge_prefill_layer_ex_kv(void* X, void* w_attn, void* Wq, void* Wk, voi
         g.ngroups = 3;
         g.Wx[0] = static_cast<const uint8_t*>(Wk); g.Yx[0] = k; g.Nx[0] = HK;
         g.Wx[1] = static_cast<const uint8_t*>(Wv); g.Yx[1] = v; g.Nx[1] = HK;
-        qr::gemm_plan(g);
-        if (qr::gemm_grouped_ok(g)) {
-            rc = check(qr::launch_gemm(g, g_stream), "layer qkv");
-        } else {
-            rc = proj(a, Wq, nullptr, q, nullptr, HQ, dm, D);
-            rc = rc ? rc : proj(a, Wk, nullptr, k, nullptr, HK, dm, D);
-            rc = rc ? rc : proj(a, Wv, nullptr, v, nullptr, HK, dm, D);
-        }
+        rc = launch(g);
     }
     if (!rc && rope) {
-        rc = check(qr::launch_rope(q, Hq, M, D, theta, offset, traditional, g_stream), "layer rope");
-        rc = rc ? rc : check(qr::launch_rope(k, Hkv, M, D, theta, offset, traditional, g_stream), "layer rope");
+        rc = check(qr::launch_rope(q, Hq, M, D, theta, offset, traditional, g_stream, k, Hkv), "layer rope");
     }
     if (!rc) {
         // The Q8_0 KV cache (unified_prefill_engine.mm:548-572), written in

@@ -173,6 +173,8 @@ gemm_rb_kernel(GemmParams p) {
             const uint32_t t1 = ntm * ((p.Nx[0] + C::BN - 1) / C::BN);
             const int gx = (bid < t1 || p.ngroups == 2) ? 0 : 1;
             if (gx == 1) bid -= t1;
+            if constexpr (SPLIT)  // the groups' partials lie one after the other
+                p.ws += (size_t)p.ksplit * p.M * (p.N + (gx == 1 ? p.Nx[0] : 0u));
             p.W = p.Wx[gx];
             p.Y = p.Yx[gx];
             p.N = p.Nx[gx];

@@ -111,8 +111,21 @@ __global__ void __launch_bounds__(gemv::kThreads, (gemv::waves_per_simd<F, NC * 
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t r16 = lane & 15, g = lane >> 4;
+    uint32_t bid = blockIdx.x;
+    if (p.ngroups > 1) {  // grouped launch: this workgroup's matrix, output and width
+        const uint32_t t0 = (p.N + CW - 1) / CW;
+        if (bid >= t0) {
+            bid -= t0;
+            const uint32_t t1 = (p.Nx[0] + CW - 1) / CW;
+            const int gx = (bid < t1 || p.ngroups == 2) ? 0 : 1;
+            if (gx == 1) bid -= t1;
+            p.W = p.Wx[gx];
+            p.Y = p.Yx[gx];
+            p.N = p.Nx[gx];
+        }
+    }
     const uint32_t M = p.M, N = p.N, K = p.K, col_bytes = (uint32_t)p.col_bytes;
-    const uint32_t n0 = blockIdx.x * CW, ncols = min((uint32_t)CW, N - n0);
+    const uint32_t n0 = bid * CW, ncols = min((uint32_t)CW, N - n0);
     const uint32_t nch = K / 256, c0 = nch * (uint32_t)wave / W, c1 = nch * (uint32_t)(wave + 1) / W;
 
     __amdgpu_buffer_rsrc_t wr[PL];
@@ -206,6 +219,7 @@ __global__ void __launch_bounds__(gemv::kThreads, (gemv::waves_per_simd<F, NC * 
 // this one):
 //  * SwiGLU: always, against the 128-row tiles (MLX, K = 4096, N = 14336:
 //    M = 1 33.2 -> 21.3, M = 16 34.0 -> 33.2);
+//  * a layer's Q, K and V in one launch: always (they were three launches);
 //  * formats without a small-M kernel: always (Q8_0 4096 x 4096, M = 1 11.1 ->
 //    6.9, M = 16 14.1 -> 9.4);
 //  * where the small-M kernel needs its K split: up to 8 rows (MLX K = 14336,
@@ -216,8 +230,8 @@ __global__ void __launch_bounds__(gemv::kThreads, (gemv::waves_per_simd<F, NC * 
 //  * where it runs as one kernel: one or two rows (MLX 4096 x 4096: M = 1
 //    5.5 -> 4.8, M = 2 5.6 -> 5.1, M = 4 5.6 -> 5.7), Q4_K up to 8 (8.2 -> 6.2).
 bool gemv_fits(const GemmParams& p) {
-    if (p.M > 16 || p.K % 256 || p.ngroups > 1) return false;
-    if (p.W2 || !skinny_supported(p)) return true;
+    if (p.M > 16 || p.K % 256) return false;
+    if (p.W2 || p.ngroups > 1 || !skinny_supported(p)) return true;
     const uint32_t tiles = (p.N + 15) / 16;
     if (skinny_one_kernel(p)) return p.M <= (p.format == QUANT_Q4_K ? 8u : 2u);
     return tiles <= 1024 && (p.M <= 8 || tiles <= 128);
@@ -227,12 +241,15 @@ template <int F>
 static hipError_t launch_gemv_f(const GemmParams& p, hipStream_t st) {
     // two column tiles per workgroup when the workgroups of one would not be
     // resident at once (MLX N = 14336, K = 4096, M = 1: 15.5 -> 12.8 us)
-    const uint32_t tiles = (p.N + 15) / 16;
-    const bool two = tiles > 512;
-    const dim3 grid(two ? (tiles + 1) / 2 : tiles), block(gemv::kThreads);
-    if (p.W2) hipLaunchKernelGGL((gemv_kernel<F, 1, 2>), dim3(tiles), block, 0, st, p);
-    else if (two) hipLaunchKernelGGL((gemv_kernel<F, 2, 1>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((gemv_kernel<F, 1, 1>), grid, block, 0, st, p);
+    auto tiles = [&](uint32_t cw) {
+        uint32_t t = (p.N + cw - 1) / cw;
+        for (uint32_t g = 1; g < p.ngroups && g < 3; g++) t += (p.Nx[g - 1] + cw - 1) / cw;
+        return t;
+    };
+    const dim3 block(gemv::kThreads);
+    if (p.W2) hipLaunchKernelGGL((gemv_kernel<F, 1, 2>), dim3(tiles(16)), block, 0, st, p);
+    else if (tiles(16) > 512) hipLaunchKernelGGL((gemv_kernel<F, 2, 1>), dim3(tiles(32)), block, 0, st, p);
+    else hipLaunchKernelGGL((gemv_kernel<F, 1, 1>), dim3(tiles(16)), block, 0, st, p);
     return hipGetLastError();
 }
 

@@ -17,10 +17,21 @@ namespace qr {
 // partials are read once, as streaming loads.
 constexpr int kRedVec = 8;
 
+// blockIdx.y is the group of a grouped projection (its partials follow the
+// previous group's).
+struct RedGroups {
+    _Float16* Y[3];
+    uint32_t N[3];
+};
+
 template <bool DUAL>
 __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float* __restrict__ ws, uint32_t ks, uint32_t M,
-                                                            uint32_t N, const _Float16* __restrict__ R,
-                                                            _Float16* __restrict__ Y, uint32_t head_D) {
+                                                            RedGroups gr, const _Float16* __restrict__ R,
+                                                            uint32_t head_D) {
+    const uint32_t grp = blockIdx.y;
+    if (grp > 0) ws += (size_t)ks * M * (gr.N[0] + (grp > 1 ? gr.N[1] : 0u));
+    const uint32_t N = grp == 0 ? gr.N[0] : (grp == 1 ? gr.N[1] : gr.N[2]);
+    _Float16* const __restrict__ Y = grp == 0 ? gr.Y[0] : (grp == 1 ? gr.Y[1] : gr.Y[2]);
     const size_t plane = (size_t)M * N;
     const size_t e0 = ((size_t)blockIdx.x * 256 + threadIdx.x) * kRedVec;
     if (e0 >= plane) return;
@@ -87,15 +98,20 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float* __restr
     }
 }
 
+static hipError_t reduce_groups(const float* ws, uint32_t ks, uint32_t M, const RedGroups& gr, uint32_t ngroups, bool dual,
+                                const _Float16* R, uint32_t head_D, hipStream_t st) {
+    uint32_t n = gr.N[0];
+    for (uint32_t g = 1; g < ngroups; g++) n = gr.N[g] > n ? gr.N[g] : n;
+    const size_t plane = (size_t)M * n;
+    const dim3 grid((unsigned)((plane + 256 * kRedVec - 1) / (256 * kRedVec)), ngroups);
+    if (dual) hipLaunchKernelGGL(splitk_reduce_kernel<true>, grid, dim3(256), 0, st, ws, ks, M, gr, R, head_D);
+    else hipLaunchKernelGGL(splitk_reduce_kernel<false>, grid, dim3(256), 0, st, ws, ks, M, gr, R, head_D);
+    return hipGetLastError();
+}
+
 hipError_t launch_splitk_reduce(const float* ws, uint32_t ks, uint32_t M, uint32_t N, bool dual, const _Float16* R,
                                 _Float16* Y, uint32_t head_D, hipStream_t st) {
-    const size_t plane = (size_t)M * N;
-    const unsigned blocks = (unsigned)((plane + 256 * kRedVec - 1) / (256 * kRedVec));
-    if (dual)
-        hipLaunchKernelGGL(splitk_reduce_kernel<true>, dim3(blocks), dim3(256), 0, st, ws, ks, M, N, R, Y, head_D);
-    else
-        hipLaunchKernelGGL(splitk_reduce_kernel<false>, dim3(blocks), dim3(256), 0, st, ws, ks, M, N, R, Y, head_D);
-    return hipGetLastError();
+    return reduce_groups(ws, ks, M, RedGroups{{Y, nullptr, nullptr}, {N, 0, 0}}, 1, dual, R, head_D, st);
 }
 
 static hipError_t launch_gemm_main(const GemmParams& p, hipStream_t st) {
@@ -116,7 +132,8 @@ static hipError_t launch_gemm_main(const GemmParams& p, hipStream_t st) {
 hipError_t launch_gemm(const GemmParams& p, hipStream_t st) {
     hipError_t e = launch_gemm_main(p, st);
     if (e == hipSuccess && p.ksplit > 1)
-        e = launch_splitk_reduce(p.ws, p.ksplit, p.M, p.N, p.W2 != nullptr, p.R, p.Y, p.head_D, st);
+        e = reduce_groups(p.ws, p.ksplit, p.M, RedGroups{{p.Y, p.Yx[0], p.Yx[1]}, {p.N, p.Nx[0], p.Nx[1]}},
+                          p.ngroups > 1 ? p.ngroups : 1, p.W2 != nullptr, p.R, p.head_D, st);
     return e;
 }
 
@@ -127,9 +144,10 @@ static uint32_t tiles_of(const GemmParams& p, const RbShape& d) {
     return T;
 }
 
-bool gemm_grouped_ok(const GemmParams& p) {
-    // the groups share the shape; the grid needs no K split
-    return p.ngroups >= 2 && p.ngroups <= 3 && !p.W2 && !p.R && p.ksplit <= 1;
+static uint32_t columns_of(const GemmParams& p) {
+    uint32_t n = p.N;
+    for (uint32_t g = 1; g < p.ngroups && g < 3; g++) n += p.Nx[g - 1];
+    return n;
 }
 
 // One workgroup fits a CU, so a grid runs in waves of 256 tiles.  What a wave
@@ -163,7 +181,7 @@ static float plan_cost(const GemmParams& p, int shape, uint32_t ks) {
     if (rem) c += w.lo + (rem > 128 ? (w.hi - w.lo) * (float)(rem - 128) / 128.0f : 0.0f);
     c *= (float)p.K / (4096.0f * (float)ks);
     // the partials' round trip (~4.5 TB/s) and the reduction kernel
-    if (ks > 1) c += 4.0f + (float)ks * (float)p.M * (float)p.N * (p.W2 ? 16.0f : 8.0f) / 4.5e6f;
+    if (ks > 1) c += 4.0f + (float)ks * (float)p.M * (float)columns_of(p) * (p.W2 ? 16.0f : 8.0f) / 4.5e6f;
     return c;
 }
 
@@ -200,7 +218,7 @@ void gemm_plan(GemmParams& p) {
 }
 
 size_t gemm_workspace_floats(const GemmParams& p) {
-    return p.ksplit > 1 ? (size_t)p.ksplit * p.M * p.N * (p.W2 != nullptr ? 2 : 1) : 0;
+    return p.ksplit > 1 ? (size_t)p.ksplit * p.M * columns_of(p) * (p.W2 != nullptr ? 2 : 1) : 0;
 }
 
 }  // namespace qr

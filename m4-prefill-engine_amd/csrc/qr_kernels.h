@@ -24,8 +24,8 @@ struct GemmParams {
     int shape;            // tile shape (gemm_plan)
     uint32_t group_m;     // row-tiles per XCD tile group (0: kernel default; gemm_plan)
     // Grouped launch: up to two more projections of the same X (same K,
-    // format, head_D; no residual, no SwiGLU, no K split) in the same grid,
-    // group g >= 1 writing Yx[g - 1] [M, Nx[g - 1]] from Wx[g - 1].
+    // format, head_D; no residual, no SwiGLU) in the same grid, group g >= 1
+    // writing Yx[g - 1] [M, Nx[g - 1]] from Wx[g - 1].
     uint32_t ngroups;     // 0 or 1: a single projection
     const uint8_t* Wx[2];
     _Float16* Yx[2];
@@ -35,8 +35,6 @@ struct GemmParams {
 // Tile shape, K split and tile order of p (before launch_gemm).
 void gemm_plan(GemmParams& p);
 hipError_t launch_gemm(const GemmParams& p, hipStream_t st);
-// Whether launch_gemm can run p's groups (ngroups >= 2) as one grid, as planned.
-bool gemm_grouped_ok(const GemmParams& p);
 size_t gemm_workspace_floats(const GemmParams& p);
 // Sums split-K partials ws [ks][dual ? 2 : 1][M][N] in split order and writes
 // the projection epilogue (SwiGLU when dual, + R, fp16, head-major when
@@ -93,7 +91,8 @@ hipError_t launch_rmsnorm(const _Float16* X, const _Float16* w, _Float16* Y, uin
 // Rotary position embedding in place on T [H, M, D] (D % 16 == 0), positions
 // offset + m, frequencies theta^(-2i/D); pairs (i, i + D/2), or (2i, 2i + 1)
 // when traditional.
+// T2 [H2, M, D], when given, is rotated in the same launch.
 hipError_t launch_rope(_Float16* T, uint32_t H, uint32_t M, uint32_t D, float theta, uint32_t offset,
-                       int traditional, hipStream_t st);
+                       int traditional, hipStream_t st, _Float16* T2 = nullptr, uint32_t H2 = 0);
 
 }  // namespace qr

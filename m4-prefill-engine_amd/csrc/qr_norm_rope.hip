@@ -69,14 +69,22 @@ __global__ void __launch_bounds__(256) rmsnorm_kernel(const _Float16* X, const _
 // precision; sin/cos of the reduced angle in fp32.  T is [H, M, D].
 constexpr uint32_t kRopeHeads = 4;
 
-__global__ void __launch_bounds__(128) rope_kernel(_Float16* T, uint32_t H, uint32_t M, uint32_t D, float theta,
-                                                   uint32_t offset, int traditional) {
+// Blocks past the head groups of T rotate T2 (a layer's K beside its Q).
+__global__ void __launch_bounds__(128) rope_kernel(_Float16* T, uint32_t H, _Float16* T2, uint32_t H2, uint32_t M,
+                                                   uint32_t D, float theta, uint32_t offset, int traditional) {
     const uint32_t half = D / 2, per_row = half / 8;
     const size_t t = (size_t)blockIdx.x * 128 + threadIdx.x;
     if (t >= (size_t)M * per_row) return;
     const uint32_t m = (uint32_t)(t / per_row);
     const uint32_t i0 = (uint32_t)(t % per_row) * 8;  // first pair index of this thread
-    const uint32_t h0 = blockIdx.y * kRopeHeads;
+    uint32_t by = blockIdx.y;
+    const uint32_t ny = (H + kRopeHeads - 1) / kRopeHeads;
+    if (by >= ny) {
+        by -= ny;
+        T = T2;
+        H = H2;
+    }
+    const uint32_t h0 = by * kRopeHeads;
     const double pos = (double)(offset + m);
     // inverse frequency of pair i0, then successive ratios theta^(-2/D)
     const double l2t = log2((double)theta);
@@ -153,12 +161,13 @@ hipError_t launch_rmsnorm(const _Float16* X, const _Float16* w, _Float16* Y, uin
 }
 
 hipError_t launch_rope(_Float16* T, uint32_t H, uint32_t M, uint32_t D, float theta, uint32_t offset,
-                       int traditional, hipStream_t st) {
+                       int traditional, hipStream_t st, _Float16* T2, uint32_t H2) {
     if (D % 16) return hipErrorInvalidValue;
     if (H == 0 || M == 0) return hipSuccess;
     const size_t threads = (size_t)M * (D / 16);
-    const dim3 grid((unsigned)((threads + 127) / 128), (H + kRopeHeads - 1) / kRopeHeads);
-    hipLaunchKernelGGL(rope_kernel, grid, dim3(128), 0, st, T, H, M, D, theta, offset, traditional);
+    const dim3 grid((unsigned)((threads + 127) / 128),
+                    (H + kRopeHeads - 1) / kRopeHeads + (T2 ? (H2 + kRopeHeads - 1) / kRopeHeads : 0));
+    hipLaunchKernelGGL(rope_kernel, grid, dim3(128), 0, st, T, H, T2, H2, M, D, theta, offset, traditional);
     return hipGetLastError();
 }
 

@@ -1017,6 +1017,30 @@ def test_prefill_layer_ex(bridge, oracle, norm_type, rope, traditional, Hq, Hkv,
     assert d <= 2 * TOL
 
 
+@pytest.mark.parametrize("fmt", [0, 2, 3])
+@pytest.mark.parametrize("M", [1, 16, 17, 77])
+def test_prefill_layer_short_prompts(bridge, oracle, fmt, M):
+    """Q, K and V as one launch: the few-row kernel (M <= 16), and above it one
+    split-K grid (d_model = 2048) whose three groups' partials follow each
+    other, with K and V heads narrower than Q's (2 heads and 1).  N(0, 0.02)
+    weights only: a V code on a rounding tie moves by 1 / 127 of its block's
+    largest value, which weights of 0.2 would amplify ten times per projection."""
+    dm, Hq, Hkv, D, Nm = 2048, 2, 1, 128, 256
+    X = synth.activations(M, dm, 271)
+    shapes = [(Hq * D, dm), (Hkv * D, dm), (Hkv * D, dm), (dm, Hq * D), (Nm, dm), (Nm, dm), (dm, Nm)]
+    Ws = [weights("quantized", fmt, n, k, 280 + i) for i, (n, k) in enumerate(shapes)]
+    w = (1 + 0.1 * np.random.default_rng(272).standard_normal(dm)).astype(np.float16)
+    out = empty16(M, dm)
+    bridge.prefill_layer_ex(dev(X), dev(w), *[dev(x) for x in Ws[:4]], dev(w), *[dev(x) for x in Ws[4:]], out, fmt, M,
+                            dm, Hq, Hkv, D, Nm, D ** -0.5, rope_offset=5)
+    bridge.synchronize()
+    ref = oracle.layer_ex(fmt, X, w, *Ws[:4], w, *Ws[4:], Hq, Hkv, D, Nm, D ** -0.5, norm_type=1, eps=1e-5, rope=True,
+                          theta=10000.0, offset=5, traditional=False)
+    # fp16 intermediates on both sides: an upstream tie moves an output by about
+    # one step, whose size follows the largest value
+    assert maxdiff(host(out), ref) <= 2 * max(TOL, float(tolerance.ulp16(np.abs(ref).max())))
+
+
 @pytest.mark.parametrize("fmt", [0, 1, 2, 3])
 @pytest.mark.parametrize("M,K,N", [(1030, 1024, 200), (2048, 2048, 512), (1024, 4096, 264)])
 def test_tall_narrow_projections(bridge, oracle, fmt, M, K, N):
