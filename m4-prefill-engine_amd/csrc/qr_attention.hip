@@ -14,11 +14,9 @@
 //    exchange with the partner lane (l ^ 32) -- no 32-lane reduction trees.
 //  * P stays in registers: the S^T accumulator of a lane already holds the
 //    8 keys that lane must supply as the B operand of O^T = V^T . P^T, given
-//    the matching key order in the V^T A-operand reads (two ds_read_b64).
+//    the matching key order of the cached V'^T.
 //  * fp32 running max / sum / output accumulators (the reference keeps
 //    S, P and O in half); the output is rounded to fp16 once.
-#include <type_traits>
-
 #include "qr_device.h"
 #include "qr_kernels.h"
 
@@ -85,7 +83,6 @@ hipError_t launch_quantize_q8_0(const _Float16* src, uint8_t* dst, size_t nblock
 // --------------------------------------------------------------------------
 // Flash attention
 // --------------------------------------------------------------------------
-constexpr int kBQ = 128;      // queries per query tile
 constexpr int kBKV = 64;      // keys per tile of the cache pass; the fp16 cache pads M to a multiple
 // The attention kernel reads a dequantized fp16 working copy of the cache: K'
 // [H, Mp, D] (row-major) and V'^T [H, D, Mp] (keys contiguous per dim), Mp = M
@@ -102,6 +99,9 @@ __device__ __forceinline__ uint32_t q8_pair(uint32_t codes, h2_t d) {
     return as_u32((as_h2(HI ? nib_pair_hi(u) : nib_pair_lo(u)) - off) * d);
 }
 
+// In V'^T the keys of every 16 are stored 0-3, 8-11, 4-7, 12-15: the order in
+// which a lane holds its P values, so its V^T fragment is one 16-byte read.
+//
 // Dequantized fp16 cache for the attention kernel, one workgroup per 64-key
 // tile of one head.  FROM_Q8: from Q8_0 blocks (half(q * half(d)), the
 // reference's dequantizer, brick4_attn_bench.mm:57-65); otherwise from fp16
@@ -194,11 +194,12 @@ __global__ void __launch_bounds__(256) kv_prep_kernel(const void* Ksrc, const vo
                                         (!FROM_Q8 && Vq) ? QS + QB + ((2 * kp + e) * NB + db) * 34 : nullptr);
             }
             uint32_t* t32 = reinterpret_cast<uint32_t*>(T);
+            const int kpos = (kp & ~6) | ((kp & 2) << 1) | ((kp & 4) >> 1);  // keys 4..7 and 8..11 of 16 swapped
 #pragma unroll
             for (int i = 0; i < 16; i++) {
                 const int dd = db * 32 + 2 * i;
-                t32[(dd * TR) / 2 + kp] = perm(w[1][i], w[0][i], 0x05040100u);
-                t32[((dd + 1) * TR) / 2 + kp] = perm(w[1][i], w[0][i], 0x07060302u);
+                t32[(dd * TR) / 2 + kpos] = perm(w[1][i], w[0][i], 0x05040100u);
+                t32[((dd + 1) * TR) / 2 + kpos] = perm(w[1][i], w[0][i], 0x07060302u);
             }
         }
     }
@@ -246,167 +247,148 @@ __global__ void __launch_bounds__(256) kv_prep_kernel(const void* Ksrc, const vo
 }
 
 // --------------------------------------------------------------------------
-// Software-pipelined causal attention over the fp16 cache, with the
-// query-tile pairing that balances the causal work: one workgroup per (light,
-// heavy) pair of 128-query tiles -- a and qtiles - 1 - a -- so every
-// workgroup carries the same work.  A key tile is 32-key units (four at D =
-// 64, two at D = 128); units whose keys all lie above a wave's diagonal are
-// skipped.
+// Causal attention over the fp16 cache.  A workgroup is 4 waves (one per SIMD;
+// two workgroups per CU, whose softmax and matrix phases overlap because no
+// barrier ties them): 4 / NK blocks of 32 queries times NK key groups, group kg
+// taking the kg-th share of every tile's 32-key units, the partial states
+// merged through LDS at the end of a query tile.  Per 32 x 32 unit a wave issues
+// D / 16 MFMAs for S^T = K . Q^T, a softmax of ~85 VALU ops and 16 exponentials
+// (16 cycles each) and D / 16 MFMAs for O^T += V^T . P^T, and reads 128 D bytes
+// of LDS; at D = 128 the three take about the same time, at D = 64 the VALU is
+// what bounds it.
 //
-// D = 64 (NG = 2, 8 waves, two per SIMD): group 0 takes the light tile's
-// queries and group 1 the heavy tile's on the key tiles both need; the heavy
-// tile's remaining key tiles go in pairs, one tile of a pair per group (a last
-// odd tile split two units per group), and group 0's partial softmax state is
-// merged into group 1's at the end.
-// D = 128 (NG = 1, 4 waves, one per SIMD, so a wave has the registers for the
-// 32 x 128 output tile and both fragment sets): the light tile's key tiles,
-// then the heavy tile's, as one stream, two tiles per barrier.
+// Key tiles of 32 KB (K rows, then V^T rows) are double-buffered in LDS, copied
+// there by buffer loads in inline asm one tile ahead; the only barrier is one
+// per tile, behind the wave's own vmcnt(0).  Units above a wave's diagonal are
+// skipped.  Softmax in log2 units with the scale folded into one fma; the
+// reference point moves lazily (only past 2^8, checked once per two units), the
+// halves of a row combined only then; fp32 state; P rounded to fp16 once, for
+// the MFMA and for the row sums alike.
 //
-// Pipelining: while the softmax of unit u runs on the VALU, the S^T = K . Q^T
-// MFMAs of unit u + 1 and the O^T += V^T . P^T MFMAs of unit u are issued from
-// the same fenced instruction sequence, so the matrix pipe and the vector ALU
-// work side by side inside every wave.  K/V tiles sit in a 4-deep LDS ring
-// (tiles t and t + 1 read, the look-ahead S reading ahead where that tile is
-// already visible, tiles t + 2 and t + 3 being written).  Arithmetic per
-// unit: log2-unit softmax with the scale folded into one fma, a lazily moved
-// reference point (threshold 2^8, decided per lane half, the halves combined
-// only when it moves), fp32 state, P rounded to fp16 for the MFMA and for the
-// row sums.
+// Before, one 8-wave workgroup per CU (4 waves at D = 128, one per SIMD) ran an
+// in-wave software pipeline of the two phases; at one wave per SIMD the compiler
+// moved the accumulators between register files (168 VALU ops per unit instead
+// of ~85) and nothing covered its waits.  us with the cache pass, before ->
+// now: D = 128, H = 32, Hkv = 8, M = 8100 974 -> 582; M = 1000 49.4 -> 27.5;
+// D = 64, H = 32, M = 2048 42.5 -> 40.3, M = 8192 433 -> 370, M = 500 19.5 -> 12.5.
 // --------------------------------------------------------------------------
-// keys per tile of the pipelined kernel: 128 at D = 64, 64 at D = 128 (the
-// 4-deep ring of K and V^T tiles then fits the LDS at either width)
-constexpr int pipe_keys(int D) { return D == 64 ? 128 : 64; }
-constexpr int kPVPad = 4;  // halfs of padding per V^T row of its LDS tiles
+constexpr int tile_keys(int D) { return D == 64 ? 128 : 64; }  // 32 KB of K and V^T per tile at either width
+constexpr int kTileBytes = 32768;
+constexpr int kLmBytes = 2048;  // row sums and maxima of the merge
 
-template <int D, int NG>  // NG: wave groups of 4 (2: the pair schedule; 1: the two tiles one after the other)
-__global__ void __launch_bounds__(256 * NG) flash_attn_pipe_kernel(AttnParams p) {
-    static_assert(D == 64 || D == 128, "chunk schedules written for D = 64 and D = 128");
-    constexpr int kPKV = pipe_keys(D), UPT = kPKV / 32;  // units (32 keys) per tile
-    // V^T rows of kPKV + 4 halfs (66 or 34 dwords): the fragment reads of
-    // lanes j and j + 16 land 32 banks apart (a 68-dword row put them on the
-    // same banks)
-    constexpr int KROW = D + 8, VROW = kPKV + kPVPad, DT = D / 32;
-    constexpr int NT = 256 * NG;
-    constexpr int KT = kPKV * KROW, VT = D * VROW, TILE = KT + VT;
-    constexpr int NBUF = 4;
-    constexpr int KCH = kPKV * (D / 8) / NT, VCH = D * (kPKV / 8) / NT;  // 16-byte chunks per thread
-    extern __shared__ __attribute__((aligned(16))) _Float16 smem[];
+// 1 KB global -> LDS copy (16 bytes per lane, lane l to lds_addr + 16 l); not
+// known to the compiler, so every reader waits for it explicitly.
+__device__ __forceinline__ void attn_copy(uint32_t lds_addr, uint32_t voff, u4_t rsrc, uint32_t soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :: "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(rsrc),
+                    "s"(__builtin_amdgcn_readfirstlane(soff)));
+}
+__device__ __forceinline__ u4_t attn_rsrc(const void* base, uint32_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    return u4_t{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a),
+                (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu),
+                (uint32_t)__builtin_amdgcn_readfirstlane(bytes), (uint32_t)kBufferFlags};
+}
+__device__ __forceinline__ float max3(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
+
+template <int D, int NK>  // NK: key groups; 4 / NK blocks of 32 queries per workgroup
+__global__ void __launch_bounds__(256, 2) flash_attn_kernel(AttnParams p, int paired) {
+    constexpr int KT = tile_keys(D), UPT = KT / 32, UW = UPT / NK, NQ = 4 / NK, BQ = 32 * NQ;
+    constexpr int DT = D / 32, KK = D / 16;
+    constexpr int KB = KT * D * 2;             // bytes of a K tile
+    constexpr int KU = D / 8, VU = KT / 8;     // 16-byte units per K row, per V^T row
+    constexpr int CPW = kTileBytes / 2 / 1024 / 4;  // copies per wave of K, and of V^T
+    constexpr int NB = UW < 2 ? 1 : 2;         // units per softmax batch
+    static_assert(KB == kTileBytes / 2 && D * KT * 2 == kTileBytes / 2, "tile bytes");
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int grp = NG == 2 ? wave >> 2 : 0, wq = wave & 3;
+    const int qb_ = wave % NQ, kg = wave / NQ;  // query block and key group
     const int g = lane >> 5, j = lane & 31;
     const int M = (int)p.M, Mp = (int)p.Mp;
-    const int qtiles = (M + kBQ - 1) / kBQ;
+    const int qtiles = (M + BQ - 1) / BQ;
     const int pr = (int)blockIdx.x / (int)p.H, h = (int)blockIdx.x % (int)p.H;
-    const int qa = pr, qb = qtiles - 1 - pr;
-    auto tiles_for = [&](int qt) { return (min((qt + 1) * kBQ, M) - 1) / kPKV + 1; };
-    const int Tl = qa == qb ? 0 : tiles_for(qa);
-    const int Th = tiles_for(qb);
+    // paired: a light and a heavy query tile; else one, the heavy half of them
+    // first, descending, then the light half, ascending (workgroups half a
+    // grid apart, which share a CU when the grid fills it twice, then add up alike)
+    const int nh = (qtiles + 1) / 2;
+    const int qz = pr < nh ? qtiles - 1 - pr : pr - nh;
+    const int qa = paired ? pr : qz;
+    auto tiles_for = [&](int qt) { return (min((qt + 1) * BQ, M) - 1) / KT + 1; };
+    const int Tl = qa == qz ? 0 : tiles_for(qa);
+    const int S = Tl + tiles_for(qz);
+    auto tile_of = [&](int s) { return s < Tl ? s : s - Tl; };
 
     const size_t head_elems = (size_t)M * D;
     const int hk = p.Hkv ? h / ((int)p.H / (int)p.Hkv) : h;
     const uint32_t cbytes = (uint32_t)((size_t)Mp * D * 2);
-    auto kr = make_rsrc(p.Kf + (size_t)hk * Mp * D, cbytes);
-    auto vr = make_rsrc(p.Vtf + (size_t)hk * Mp * D, cbytes);
-    auto qr_ = make_rsrc(p.Q + (size_t)h * head_elems, (uint32_t)(head_elems * 2));
+    const u4_t kr = attn_rsrc(p.Kf + (size_t)hk * Mp * D, cbytes);
+    const u4_t vr = attn_rsrc(p.Vtf + (size_t)hk * Mp * D, cbytes);
+    const auto qr_ = make_rsrc(p.Q + (size_t)h * head_elems, (uint32_t)(head_elems * 2));
 
-    // ---- K / V^T tiles: fetched 3 tiles ahead into registers, written to
-    // the LDS ring 2 tiles ahead.  Keys past Mp read zeros: for K the offset
-    // runs past the head's cache, for V^T (rows of Mp keys per dim) a chunk
-    // past Mp would be the next dim's first keys, so its offset is made
-    // out of range -- a masked key must not carry an inf or NaN into P V. ----
-    // V^T chunk c of a tile (16 bytes: 8 keys of one dim row).  An 8-byte
-    // LDS write pass serves 16 lanes on the 32 banks; at D = 64 (16 chunks per
-    // 66-dword row) 16 chunks of one row would put chunks k and k + 8 on the
-    // same banks, so a pass takes 8 chunks each of two adjacent rows (the
-    // second row lands 2 banks over).  At D = 128 (8 chunks per row) one pass
-    // already spans two rows.
-    auto vchunk = [&](int c, int& row, int& ch) {
-        constexpr int CPR = kPKV / 8;
-        if constexpr (CPR == 16) {
-            const int b = c >> 4, l = c & 15;
-            row = 2 * (b >> 1) + (l >> 3);
-            ch = 8 * (b & 1) + (l & 7);
-        } else {
-            row = c / CPR;
-            ch = c % CPR;
+    // ---- tile copies.  K rows (keys) hold KU 16-byte units, V^T rows (dims) VU;
+    // unit u of row r sits at u ^ swz, which depends on r mod 32 only and puts
+    // the 16 rows of a fragment-read pass on distinct banks ----
+    auto swz = [](int units, uint32_t r) -> uint32_t {
+        r &= 31u;
+        return units == 16 ? (r & 15u) : ((r ^ (r >> 3)) & 7u);
+    };
+    uint32_t ko[CPW], vo[CPW], vk[CPW];
+#pragma unroll
+    for (int q = 0; q < CPW; q++) {
+        const uint32_t un = 64u * (uint32_t)(CPW * wave + q) + (uint32_t)lane;
+        const uint32_t kr_ = un / KU, ku = (un % KU) ^ swz(KU, kr_);
+        ko[q] = (kr_ * D + 8u * ku) * 2u;
+        const uint32_t vr_ = un / VU, vu = (un % VU) ^ swz(VU, vr_);
+        vk[q] = 8u * vu;
+        vo[q] = (vr_ * (uint32_t)Mp + 8u * vu) * 2u;
+    }
+    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)smem);
+    auto issue = [&](int s) {
+        const uint32_t k0 = (uint32_t)(tile_of(s) * KT);
+        const uint32_t dst = lds0 + (uint32_t)(s & 1) * kTileBytes + (uint32_t)(CPW * wave) * 1024u;
+        const bool part = k0 + KT > (uint32_t)Mp;  // a V^T chunk past Mp would be the next dim's first keys
+#pragma unroll
+        for (int q = 0; q < CPW; q++) {
+            attn_copy(dst + q * 1024u, ko[q] + k0 * D * 2u, kr, 0);  // rows past Mp: past the head's cache
+            attn_copy(dst + KB + q * 1024u, part && k0 + vk[q] >= (uint32_t)Mp ? kOOB : vo[q], vr, k0 * 2u);
         }
     };
-    struct Raw { u4_t k[KCH], v[VCH]; };
-    auto fetch = [&](int t, Raw& r) {
-        const int k0 = t * kPKV;
-#pragma unroll
-        for (int i = 0; i < KCH; i++) {
-            const int c = tid + NT * i;
-            r.k[i] = ld_b128(kr, (uint32_t)((k0 + c / (D / 8)) * D + (c % (D / 8)) * 8) * 2u);
-        }
-#pragma unroll
-        for (int i = 0; i < VCH; i++) {
-            int vrow, vch;
-            vchunk(tid + NT * i, vrow, vch);
-            const int key = k0 + vch * 8;  // Mp is a multiple of 8: whole chunks in or out
-            r.v[i] = ld_b128(vr, key < Mp ? (uint32_t)(vrow * Mp + key) * 2u : kOOB);
-        }
-    };
-    auto kbuf = [&](int slot) { return smem + slot * TILE; };
-    auto vbuf = [&](int slot) { return smem + slot * TILE + KT; };
-    auto stage = [&](const Raw& r, int slot) {
-#pragma unroll
-        for (int i = 0; i < KCH; i++) {
-            const int c = tid + NT * i;
-            *reinterpret_cast<u4_t*>(kbuf(slot) + (c / (D / 8)) * KROW + (c % (D / 8)) * 8) = r.k[i];
-        }
-#pragma unroll
-        for (int i = 0; i < VCH; i++) {
-            int vrow, vch;
-            vchunk(tid + NT * i, vrow, vch);
-            _Float16* dst = vbuf(slot) + vrow * VROW + vch * 8;
-            if constexpr (VROW % 8 == 0) {
-                *reinterpret_cast<u4_t*>(dst) = r.v[i];
-            } else {  // rows 8-byte aligned only
-                reinterpret_cast<u2_t*>(dst)[0] = u2_t{r.v[i].x, r.v[i].y};
-                reinterpret_cast<u2_t*>(dst)[1] = u2_t{r.v[i].z, r.v[i].w};
-            }
-        }
-    };
-
-    // ---- this wave's units (key start 32 * unit index within the keys):
-    // segment 1 = units 0..3 of tiles [0, Tl) (light queries for group 0,
-    // heavy for group 1); segment 2 = tiles [Tl, Th) on the heavy queries, in
-    // pairs (group 0 the first tile of a pair, group 1 the second, all four
-    // units) and, when their count is odd, a last tile split two units per
-    // group.  Each keeps the units whose first key is at or below the wave's
-    // last query (n1: group 0's light units). ----
-    const int qwL = qa * kBQ + wq * 32, qwH = qb * kBQ + wq * 32;
-    const int n1 = grp == 0 ? (Tl > 0 ? min(UPT * Tl, (qwL + 31) / 32 + 1) : 0) : UPT * Tl;
 
     float c = p.scale * 1.4426950408889634f;  // log2 units
     const bool neg = c < 0.0f;
     if (neg) c = -c;
 
-    h8_t qf[D / 16];
-    auto load_q = [&](int qw, h8_t* dst) {
+    // fragment offsets in a tile: K row 32 u + j, unit 2 kk + g; V^T row 32 t + j,
+    // unit 4 u + 2 t2 + g, for this wave's units u = kg UW + b
+    uint32_t kof[KK], vof[UW * 2];
 #pragma unroll
-        for (int kk = 0; kk < D / 16; kk++) {
-            const int my_q = qw + j;
-            const uint32_t off = my_q < M ? ((uint32_t)my_q * D + kk * 16 + 8 * g) * 2u : kOOB;
-            dst[kk] = __builtin_bit_cast(h8_t, ld_b128(qr_, off));
-            if (neg) dst[kk] = -dst[kk];
-        }
-    };
-    // group 0 starts on the light queries when it has any, else on the heavy ones
-    bool light = grp == 0 && n1 > 0;
-    int qw = light ? qwL : qwH;
-    load_q(qw, qf);
+    for (int kk = 0; kk < KK; kk++) kof[kk] = (uint32_t)j * (KU * 16u) + 16u * ((uint32_t)(2 * kk + g) ^ swz(KU, (uint32_t)j));
+#pragma unroll
+    for (int x = 0; x < UW * 2; x++)
+        vof[x] = (uint32_t)j * (VU * 16u) + 16u * ((uint32_t)(4 * kg * UW + 2 * x + g) ^ swz(VU, (uint32_t)j));
 
-    float m_run = -INFINITY;
-    float l_run = 0.0f;  // this lane's half of the row sum of P
+    h8_t qf[KK];
     f16v_t o[DT];
+    float m_run, l_run;  // l_run: this lane's half of the row sum of P
+    int qw = 0;
+    auto start = [&](int qt) {
+        qw = qt * BQ + qb_ * 32;
+        const int my_q = qw + j;
 #pragma unroll
-    for (int t = 0; t < DT; t++) o[t] = f16v_t{};
-    const h2_t one2 = {(_Float16)1.0f, (_Float16)1.0f};
-
-    auto store = [&](float inv) {
+        for (int kk = 0; kk < KK; kk++) {
+            const uint32_t off = my_q < M ? ((uint32_t)my_q * D + kk * 16 + 8 * g) * 2u : kOOB;
+            qf[kk] = __builtin_bit_cast(h8_t, ld_b128(qr_, off));
+            if (neg) qf[kk] = -qf[kk];
+        }
+        m_run = -INFINITY;
+        l_run = 0.0f;
+#pragma unroll
+        for (int t = 0; t < DT; t++) o[t] = f16v_t{};
+    };
+    auto store = [&]() {
+        const float l = l_run + __shfl_xor(l_run, 32);
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
         const int my_q = qw + j;
         if (my_q >= M) return;
 #pragma unroll
@@ -423,393 +405,183 @@ __global__ void __launch_bounds__(256 * NG) flash_attn_pipe_kernel(AttnParams p)
             }
     };
 
-    // ---- one unit: S^T of unit (slot, hh) is in s_in; the look-ahead unit's
-    // S^T (ring slot nsl, unit hn) is computed into s_out beside the softmax;
-    // MASK applies the causal / length mask to s_in first ----
-    const int kbase = j * KROW + 8 * g, vbase = j * VROW + 4 * g;
-    auto unit_core = [&](int slot, int hh, int key0, bool mask, f16v_t& s_in, int nsl, int hn, f16v_t& s_out) {
-        if (mask) {
-            const int my_q = qw + j;
+    // ---- this wave's units b0 .. b0 + NB - 1 of the tile in `buf` (first key
+    // key0), the first `live` of them at or below its last query ----
+    const h2_t one2 = {(_Float16)1.0f, (_Float16)1.0f};
+    auto batch = [&](const uint8_t* buf, int b0, int key0, int live) {
+        f16v_t s[NB];
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int key = key0 + 8 * (r >> 2) + 4 * g + (r & 3);
-                s_in[r] = (key <= my_q && key < M) ? s_in[r] : -INFINITY;
+        for (int b = 0; b < NB; b++) {
+            if (b >= live) break;
+            const uint8_t* kb = buf + (kg * UW + b0 + b) * 32 * (KU * 16);
+            s[b] = f16v_t{};
+#pragma unroll
+            for (int kk = 0; kk < KK; kk++)
+                s[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const h8_t*>(kb + kof[kk]), qf[kk], s[b], 0, 0, 0);
+        }
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            if (b >= live) break;
+            const int k0 = key0 + 32 * b;
+            if (k0 + 31 > qw || k0 + 31 >= M) {  // the diagonal, or the end of the keys
+                const int my_q = qw + j;
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int key = k0 + 8 * (r >> 2) + 4 * g + (r & 3);
+                    s[b][r] = (key <= my_q && key < M) ? s[b][r] : -INFINITY;
+                }
             }
         }
-        // V^T fragments of this unit, K fragments of the look-ahead unit
-        // (at D = 128 the second halves are read inside the chunk schedule,
-        // once the registers of the first halves are free)
-        u4_t va[2][DT];
-        const _Float16* Vb = smem + slot * TILE + KT + hh * 32 + vbase;
-        auto read_va = [&](int t2) {
+        // Row maximum of each lane's half decides whether the reference point
+        // must move (by more than 2^8); only then are the halves combined.
+        float mx[4];
 #pragma unroll
-            for (int tt = 0; tt < DT; tt++) {
-                const _Float16* row = Vb + tt * 32 * VROW + t2 * 16;
-                const u2_t lo = *reinterpret_cast<const u2_t*>(row);
-                const u2_t hi = *reinterpret_cast<const u2_t*>(row + 8);
-                va[t2][tt] = u4_t{lo.x, lo.y, hi.x, hi.y};
-            }
-        };
-        h8_t kn_[D / 16];
-        const _Float16* Kb = smem + nsl * TILE + hn * 32 * KROW + kbase;
-        auto read_kn = [&](int kk0, int kk1) {
+        for (int q = 0; q < 4; q++) mx[q] = fmaxf(max3(s[0][4 * q], s[0][4 * q + 1], s[0][4 * q + 2]), s[0][4 * q + 3]);
+        if (NB > 1 && live > 1) {
 #pragma unroll
-            for (int kk = kk0; kk < kk1; kk++) kn_[kk] = *reinterpret_cast<const h8_t*>(Kb + kk * 16);
-        };
-        read_va(0);
-        if constexpr (D == 64) {
-            read_va(1);
-            read_kn(0, D / 16);
-        } else {
-            read_kn(0, 4);
+            for (int q = 0; q < 4; q++)
+                mx[q] = max3(max3(mx[q], s[NB - 1][4 * q], s[NB - 1][4 * q + 1]), s[NB - 1][4 * q + 2], s[NB - 1][4 * q + 3]);
         }
-        // Row maximum: each lane's half (16 keys) decides whether the shared
-        // reference point must move; only then are the two halves combined.
-        float mx[4];  // a shallow tree of three-input maxima
-#pragma unroll
-        for (int q = 0; q < 4; q++) mx[q] = fmaxf(fmaxf(s_in[4 * q], s_in[4 * q + 1]), fmaxf(s_in[4 * q + 2], s_in[4 * q + 3]));
-        const float hmax = fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]));
-        const float m_cand = hmax * c;
+        const float m_cand = fmaxf(max3(mx[0], mx[1], mx[2]), mx[3]) * c;
         if (__any(m_cand > m_run + 8.0f)) {
             const float m_new = fmaxf(m_run, fmaxf(m_cand, __shfl_xor(m_cand, 32)));
             const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
             m_run = m_new;
 #pragma unroll
-            for (int tt = 0; tt < DT; tt++)
+            for (int t = 0; t < DT; t++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) o[tt][r] *= alpha;
+                for (int r = 0; r < 16; r++) o[t][r] *= alpha;
             l_run *= alpha;
         }
-        // --- fenced chunks: look-ahead S MFMAs and this unit's O MFMAs
-        // interleaved with this unit's exponentials ---
-        uint32_t pk[8];
-        float e[16];
-        auto exps = [&](int r0) {  // exp2 of accumulator rows r0 .. r0 + 3
+        // raised wave priority over the exponentials and their MFMAs: the SIMD's
+        // other wave, in its S phase, yields (M = 8100, D = 128 596 -> 585 us)
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int r = r0; r < r0 + 4; r++)
-                e[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s_in[r], c, -m_run));
-        };
-        auto cvts = [&](int r0) {  // P (fp16 pairs) of rows r0 .. r0 + 3
+        for (int b = 0; b < NB; b++) {
+            if (b >= live) break;
+            uint32_t pk[8];
 #pragma unroll
-            for (int r = r0; r < r0 + 4; r += 2) {
-                const h2_t pp = __builtin_convertvector((f2_t){e[r], e[r + 1]}, h2_t);
+            for (int r = 0; r < 16; r += 2) {
+                const f2_t e = {__builtin_amdgcn_exp2f(__builtin_fmaf(s[b][r], c, -m_run)),
+                                __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][r + 1], c, -m_run))};
+                const h2_t pp = __builtin_convertvector(e, h2_t);
                 pk[r >> 1] = as_u32(pp);
                 l_run = __builtin_amdgcn_fdot2(pp, one2, l_run, false);  // row sum of the rounded P
             }
-        };
-        auto pv = [&](int t2, int tt) {
-            const h8_t b = __builtin_bit_cast(h8_t, u4_t{pk[4 * t2], pk[4 * t2 + 1], pk[4 * t2 + 2], pk[4 * t2 + 3]});
-            o[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8_t, va[t2][tt]), b, o[tt], 0, 0, 0);
-        };
-        auto smf = [&](int kk) {  // look-ahead S^T MFMA over d = 16 kk .. 16 kk + 15
-            s_out = __builtin_amdgcn_mfma_f32_32x32x16_f16(kn_[kk], qf[kk], kk ? s_out : f16v_t{}, 0, 0, 0);
-        };
-        // raised wave priority for the interleaved block: the SIMD's other
-        // wave (in its row-max / fragment-read phase) yields issue slots to it
-        __builtin_amdgcn_s_setprio(1);
-        // each exponential is converted one chunk after it is issued, and each
-        // O MFMA follows the conversions it needs by a chunk where possible
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (D == 64) {
-            smf(0);
-            exps(0);
-            __builtin_amdgcn_sched_barrier(0);
-            smf(1);
-            exps(4);
-            cvts(0);
-            __builtin_amdgcn_sched_barrier(0);
-            smf(2);
-            exps(8);
-            cvts(4);
-            __builtin_amdgcn_sched_barrier(0);
-            smf(3);
-            pv(0, 0);
-            exps(12);
-            cvts(8);
-            __builtin_amdgcn_sched_barrier(0);
-            pv(0, 1);
-            cvts(12);
-            __builtin_amdgcn_sched_barrier(0);
-            pv(1, 0);
-            pv(1, 1);
-        } else {  // D = 128: twice the MFMAs per unit against the same softmax
-            smf(0);
-            smf(1);
-            exps(0);
-            __builtin_amdgcn_sched_barrier(0);
-            smf(2);
-            smf(3);
-            exps(4);
-            cvts(0);
-            read_kn(4, 8);
-            __builtin_amdgcn_sched_barrier(0);
-            smf(4);
-            smf(5);
-            exps(8);
-            cvts(4);
-            __builtin_amdgcn_sched_barrier(0);
-            smf(6);
-            smf(7);
-            pv(0, 0);
-            pv(0, 1);
-            exps(12);
-            cvts(8);
-            read_va(1);
-            __builtin_amdgcn_sched_barrier(0);
-            pv(0, 2);
-            pv(0, 3);
-            cvts(12);
-            __builtin_amdgcn_sched_barrier(0);
-            pv(1, 0);
-            pv(1, 1);
-            pv(1, 2);
-            pv(1, 3);
+            const uint8_t* vb = buf + KB;
+#pragma unroll
+            for (int t2 = 0; t2 < 2; t2++) {
+                const h8_t pf = __builtin_bit_cast(h8_t, u4_t{pk[4 * t2], pk[4 * t2 + 1], pk[4 * t2 + 2], pk[4 * t2 + 3]});
+#pragma unroll
+                for (int t = 0; t < DT; t++) {
+                    const h8_t va = *reinterpret_cast<const h8_t*>(vb + t * 32 * (VU * 16) + vof[2 * (b0 + b) + t2]);
+                    o[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pf, o[t], 0, 0, 0);
+                }
+            }
         }
-        __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(0);
     };
-    auto scores_now = [&](int slot, int hh, f16v_t& s) {
-        const _Float16* Kb = smem + slot * TILE + hh * 32 * KROW + kbase;
-        h8_t ka[D / 16];
-#pragma unroll
-        for (int kk = 0; kk < D / 16; kk++) ka[kk] = *reinterpret_cast<const h8_t*>(Kb + kk * 16);
-        s = f16v_t{};
-#pragma unroll
-        for (int kk = 0; kk < D / 16; kk++) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[kk], qf[kk], s, 0, 0, 0);
-    };
-    auto switch_to_heavy = [&]() {  // light queries done: write them, take the heavy ones
-        store(1.0f / (l_run + __shfl_xor(l_run, 32)));
-        light = false;
-        qw = qwH;
-        load_q(qwH, qf);
-        m_run = -INFINITY;
-        l_run = 0.0f;
-#pragma unroll
-        for (int tt = 0; tt < DT; tt++) o[tt] = f16v_t{};
-    };
 
-    // ---- main loop.  Invariant at the start of a step at tile t: tiles t and
-    // t + 1 are staged in ring slots t % 4, (t + 1) % 4 and visible, and `raw`
-    // holds tile t + 2.  A single step (segment 1, or a last odd tile of
-    // segment 2) stages t + 2, fetches t + 3 and takes tile t: group 0 the light
-    // queries (then the heavy ones), group 1 the heavy ones, four units each;
-    // on the last odd tile of segment 2 each group takes two units.  A double
-    // step (segment 2) takes tiles t and t + 1: group 0 all units of tile t,
-    // group 1 all units of tile t + 1 (heavy queries), and stages t + 2 and
-    // t + 3, so a barrier serves eight units per wave instead of four.  Every
-    // slot written held a tile finished before an earlier barrier.  The
-    // look-ahead S MFMAs go into the next tile where that tile is already
-    // visible: not across a double step's end, nor for group 1 into segment 2. ----
-    int k = 0;          // light units done (group 0, segment 1)
-    bool have = false;  // sA holds S^T of this wave's next unit
-    f16v_t sA, sB;
-    // units u0 .. u0 + nu - 1 of tile t whose first key is at or below the wave's heavy queries
-    auto units_heavy = [&](int t, int u0, int nu) {
-        int n = 0;
+    // ---- merge of the key groups' partial states through the tile buffer that
+    // every wave has finished reading (after a barrier): group 0 takes the others in order ----
+    auto merge = [&](uint8_t* buf) {
+        float* const lm = reinterpret_cast<float*>(smem + 2 * kTileBytes);
+        const int slot = (kg - 1) * NQ + qb_;
+        if (kg > 0) {
+            float* x = reinterpret_cast<float*>(buf) + slot * (DT * 16 * 64);
 #pragma unroll
-        for (int u = 0; u < UPT; u++) n += (u >= u0 && u < u0 + nu && t * kPKV + u * 32 <= qwH + 31) ? 1 : 0;
-        return n;
-    };
-    const int Tdbl = Tl + ((Th - Tl) & ~1);  // double steps over [Tl, Tdbl); a single split step at Tdbl if odd
-    // this wave's units in single-step tile t, and the first of them
-    auto count_single = [&](int t) {
-        if (t < Tl) return grp == 0 ? min(max(n1 - UPT * t, 0), UPT) : units_heavy(t, 0, UPT);
-        return units_heavy(t, grp * (UPT / 2), UPT / 2);
-    };
-    auto first_single = [&](int t) { return t < Tl ? 0 : grp * (UPT / 2); };
-
-    // cnt units of tile t (ring slot `slot`) from unit h0, S^T of the first in
-    // sA when `have`; the last unit's look-ahead goes to (s_next, h_next) when next_ok
-    auto run_tile = [&](int t, int slot, int cnt, int h0, bool next_ok, int s_next, int h_next) {
-        if (cnt == 0) return;
-        const int key_t = t * kPKV;
-        const bool full = cnt == ((NG == 2 && t >= Tdbl && t >= Tl) ? UPT / 2 : UPT) && cnt >= 2;
-        const bool unmasked = key_t + kPKV - 1 <= qw && key_t + kPKV <= M;
-        if (full && unmasked) {
-            // fast path: straight-line units, scores ping-ponging between sA and sB
-            if (!have) scores_now(slot, h0, sA);
-            const int sn = next_ok ? s_next : slot, hn = next_ok ? h_next : h0;
-            if (UPT == 4 && cnt == 4) {
-                unit_core(slot, h0, 0, false, sA, slot, h0 + 1, sB);
-                unit_core(slot, h0 + 1, 0, false, sB, slot, h0 + 2, sA);
-                unit_core(slot, h0 + 2, 0, false, sA, slot, h0 + 3, sB);
-                unit_core(slot, h0 + 3, 0, false, sB, sn, hn, sA);
-            } else {
-                unit_core(slot, h0, 0, false, sA, slot, h0 + 1, sB);
-                unit_core(slot, h0 + 1, 0, false, sB, sn, hn, sA);
-            }
-            have = next_ok;
-        } else {
-            // general path: up to four units, each with the mask where needed
-#pragma unroll
-            for (int u = 0; u < UPT; u++) {
-                if (u < cnt) {
-                    const int hh = h0 + u;
-                    if (!have) scores_now(slot, hh, sA);
-                    const bool last = u + 1 == cnt;
-                    const int nsl = last ? (next_ok ? s_next : slot) : slot;
-                    const int hn = last ? (next_ok ? h_next : hh) : hh + 1;
-                    const int key0 = key_t + hh * 32;
-                    unit_core(slot, hh, key0, key0 + 31 > qw || key0 + 31 >= M, sA, nsl, hn, sB);
-                    sA = sB;
-                    have = !last || next_ok;
-                }
-            }
-        }
-    };
-
-    if constexpr (NG == 1) {
-        // One group: the light tile's key tiles [0, Tl), then the heavy tile's
-        // [0, Th), as one stream of Tl + Th steps through the ring (the first
-        // Tl tiles are fetched twice).  Each wave switches to the heavy
-        // queries after its last light unit and idles until step Tl.
-        const int S = Tl + Th;
-        auto tile_of = [&](int s) { return s < Tl ? s : s - Tl; };
-        auto count_at = [&](int s) {
-            return s < Tl ? min(max(n1 - UPT * s, 0), UPT) : units_heavy(s - Tl, 0, UPT);
-        };
-        Raw raw;
-        fetch(tile_of(0), raw);
-        stage(raw, 0);
-        fetch(tile_of(1), raw);
-        stage(raw, 1);
-        fetch(tile_of(2), raw);
-        __syncthreads();
-        // step s: the units of tile_of(s); la: tile s + 1 is visible (look-ahead allowed)
-        auto do_step = [&](int s, bool la) {
-            const int cnt = count_at(s);
-            const bool set_ends = light && s < Tl && k + cnt == n1;
-            const bool next_ok = la && !set_ends && s + 1 < S && count_at(s + 1) > 0;
-            run_tile(tile_of(s), s & 3, cnt, 0, next_ok, (s + 1) & 3, 0);
-            if (s < Tl) k += cnt;
-            if (set_ends) switch_to_heavy();
-        };
-        // Invariant at the start of an iteration at s: steps s and s + 1 are
-        // staged and visible, `raw` holds s + 2.  Two steps per barrier: s + 2
-        // is staged first, s + 3 after both steps (its slot held s - 1).
-        for (int s = 0; s < S;) {
-            const bool dbl = s + 1 < S;
-            if (s + 2 < S) stage(raw, (s + 2) & 3);
-            if (s + 3 < S) fetch(tile_of(s + 3), raw);
-            do_step(s, true);
-            if (dbl) {
-                do_step(s + 1, false);
-                if (s + 3 < S) stage(raw, (s + 3) & 3);
-                if (s + 4 < S) fetch(tile_of(s + 4), raw);
-            }
-            __syncthreads();
-            s += dbl ? 2 : 1;
-        }
-        const float l = l_run + __shfl_xor(l_run, 32);
-        store(l > 0.0f ? 1.0f / l : 0.0f);
-    } else {
-        // ---- prologue ----
-        Raw raw;
-        fetch(0, raw);
-        stage(raw, 0);
-        fetch(1, raw);
-        stage(raw, 1);
-        fetch(2, raw);
-        __syncthreads();
-
-        int t = 0;
-        while (t < Th) {
-            const bool dbl = t >= Tl && t < Tdbl;
-            if (t + 2 < Th) stage(raw, (t + 2) & 3);
-            if (t + 3 < Th) fetch(t + 3, raw);  // double step: staged at its end
-            int mt = t, cnt, h0 = 0, h_next = 0;
-            bool next_ok = false, set_ends = false;
-            if (!dbl) {
-                cnt = count_single(t);
-                h0 = first_single(t);
-                // look-ahead of the tile's last unit: this wave's first unit of the
-                // next step, when that step starts it at tile t + 1 (visible) with the
-                // same queries
-                set_ends = light && k + cnt == n1;
-                if (!set_ends && t + 1 < Th) {
-                    if (t + 1 < Tl || t + 1 >= Tdbl) {
-                        next_ok = count_single(t + 1) > 0;
-                        h_next = first_single(t + 1);
-                    } else if (grp == 0) {  // next: a double step, whose first tile is group 0's
-                        next_ok = units_heavy(t + 1, 0, UPT) > 0;
-                    }
-                }
-            } else {
-                mt = t + grp;  // this group's tile of the pair
-                cnt = units_heavy(mt, 0, UPT);
-            }
-            run_tile(mt, mt & 3, cnt, h0, next_ok, (t + 1) & 3, h_next);
-            if (!dbl) {
-                if (t < Tl && grp == 0) k += cnt;
-                if (set_ends) switch_to_heavy();
-            } else {
-                if (t + 3 < Th) stage(raw, (t + 3) & 3);
-                if (t + 4 < Th) fetch(t + 4, raw);
-            }
-            __syncthreads();
-            t += dbl ? 2 : 1;
-        }
-
-        // ---- merge group 0's partial state for the heavy queries into group 1's ----
-        // One record of DT * 16 + 2 floats per lane (o, l, m), padded to a
-        // multiple of 4 floats and written as 16-byte vectors: a lane stride
-        // of 4 (mod 8) dwords puts the 16 lanes of a vector access on
-        // distinct banks.
-        constexpr int SW = (DT * 16 + 2 + 3) / 4 * 4 + ((((DT * 16 + 2 + 3) / 4) & 1) ? 0 : 4);
-        float* X = reinterpret_cast<float*>(smem);
-        static_assert(4 * 64 * SW * 4 <= NBUF * TILE * 2, "merge buffer fits the tile ring");
-        float* x = X + (wq * 64 + lane) * SW;
-        if (grp == 0) {
-    #pragma unroll
             for (int t = 0; t < DT; t++)
-    #pragma unroll
+#pragma unroll
                 for (int r = 0; r < 16; r += 4)
-                    *reinterpret_cast<f4_t*>(x + t * 16 + r) = f4_t{o[t][r], o[t][r + 1], o[t][r + 2], o[t][r + 3]};
-            *reinterpret_cast<f2_t*>(x + DT * 16) = f2_t{l_run, m_run};
+                    *reinterpret_cast<f4_t*>(x + ((t * 4 + r / 4) * 64 + lane) * 4) = f4_t{o[t][r], o[t][r + 1], o[t][r + 2], o[t][r + 3]};
+            *reinterpret_cast<f2_t*>(lm + (slot * 64 + lane) * 2) = f2_t{l_run, m_run};
         }
         __syncthreads();
-        if (grp == 1) {
-            const f2_t lm = *reinterpret_cast<const f2_t*>(x + DT * 16);
-            const float ma = lm.y;
-            const float m = fmaxf(ma, m_run);
-            const float fa = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ma - m);
-            const float fb = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m);
-    #pragma unroll
-            for (int t = 0; t < DT; t++)
-    #pragma unroll
-                for (int r = 0; r < 16; r += 4) {
-                    const f4_t v = *reinterpret_cast<const f4_t*>(x + t * 16 + r);
-                    o[t][r] = o[t][r] * fb + v.x * fa;
-                    o[t][r + 1] = o[t][r + 1] * fb + v.y * fa;
-                    o[t][r + 2] = o[t][r + 2] * fb + v.z * fa;
-                    o[t][r + 3] = o[t][r + 3] * fb + v.w * fa;
-                }
-            const float lh = l_run * fb + lm.x * fa;
-            const float l = lh + __shfl_xor(lh, 32);
-            store(l > 0.0f ? 1.0f / l : 0.0f);
+        if (kg == 0) {
+#pragma unroll 1
+            for (int k = 1; k < NK; k++) {
+                const int sl = (k - 1) * NQ + qb_;
+                const float* x = reinterpret_cast<const float*>(buf) + sl * (DT * 16 * 64);
+                const f2_t q = *reinterpret_cast<const f2_t*>(lm + (sl * 64 + lane) * 2);
+                const float m = fmaxf(q.y, m_run);
+                const float fa = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(q.y - m);
+                const float fb = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m);
+#pragma unroll
+                for (int t = 0; t < DT; t++)
+#pragma unroll
+                    for (int r = 0; r < 16; r += 4) {
+                        const f4_t v = *reinterpret_cast<const f4_t*>(x + ((t * 4 + r / 4) * 64 + lane) * 4);
+                        o[t][r] = o[t][r] * fb + v.x * fa;
+                        o[t][r + 1] = o[t][r + 1] * fb + v.y * fa;
+                        o[t][r + 2] = o[t][r + 2] * fb + v.z * fa;
+                        o[t][r + 3] = o[t][r + 3] * fb + v.w * fa;
+                    }
+                l_run = l_run * fb + q.x * fa;
+                m_run = m;
+            }
+        }
+    };
+
+    // ---- one stream of tiles: the light query tile's, then the heavy one's ----
+    start(Tl > 0 ? qa : qz);
+    issue(0);
+    for (int s = 0; s < S; s++) {
+        if (s == Tl && s > 0) start(qz);
+        // own copies of step s have landed, every wave is past step s - 1
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (s + 1 < S) issue(s + 1);
+        uint8_t* const buf = smem + (s & 1) * kTileBytes;
+        const int key_t = tile_of(s) * KT;
+#pragma unroll
+        for (int b = 0; b < UW; b += NB) {
+            const int key0 = key_t + 32 * (kg * UW + b);
+            const int live = key0 > qw + 31 ? 0 : (NB > 1 && key0 + 32 <= qw + 31 ? NB : 1);
+            if (live > 0) batch(buf, b, key0, live);
+        }
+        if (s == Tl - 1 || s == S - 1) {
+            if constexpr (NK > 1) {
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                merge(buf);
+            }
+            if (kg == 0) store();
         }
     }
 }
-// LDS of the pipelined kernel: the 4-deep ring of K [key][D + 8] and V^T [D][key + 4] tiles
-constexpr size_t pipe_lds(int D) { return 4 * (size_t)(pipe_keys(D) * (D + 8) + D * (pipe_keys(D) + kPVPad)) * 2; }
 
-template <int D, int NG>
-static hipError_t launch_pipe(const AttnParams& p, hipStream_t st) {
-    const uint32_t qtiles = (p.M + kBQ - 1) / kBQ;  // a workgroup takes a light and a heavy query tile
-    static size_t attr[kMaxDevices] = {};  // the tile ring needs more than the default 64 KB of LDS
-    const hipError_t e = lds_limit_once((const void*)flash_attn_pipe_kernel<D, NG>, pipe_lds(D), attr);
+template <int D, int NK>
+static hipError_t launch_attn(const AttnParams& p, int paired, hipStream_t st) {
+    constexpr uint32_t bq = 128 / NK;
+    constexpr size_t lds = 2 * kTileBytes + kLmBytes;
+    const uint32_t qtiles = (p.M + bq - 1) / bq;
+    static size_t attr[kMaxDevices] = {};  // more than the default 64 KB of LDS
+    const hipError_t e = lds_limit_once((const void*)flash_attn_kernel<D, NK>, lds, attr);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((flash_attn_pipe_kernel<D, NG>), dim3(((qtiles + 1) / 2) * p.H), dim3(256 * NG), pipe_lds(D), st, p);
+    hipLaunchKernelGGL((flash_attn_kernel<D, NK>), dim3((paired ? (qtiles + 1) / 2 : qtiles) * p.H), dim3(256), lds, st, p, paired);
     return hipGetLastError();
 }
 
 hipError_t launch_flash_attn_q8_0(const AttnParams& p, hipStream_t st) {
     // the kernels read the dequantized fp16 cache (launch_kv_prep)
     if (p.Kf == nullptr || p.Vtf == nullptr || p.Mp < p.M || p.Mp % kBKV) return hipErrorInvalidValue;
-    switch (p.D) {
-        case 64: return launch_pipe<64, 2>(p, st);
-        case 128: return launch_pipe<128, 1>(p, st);
-        default: return hipErrorInvalidValue;
+    if (p.D != 64 && p.D != 128) return hipErrorInvalidValue;
+    auto qtiles = [&](uint32_t nk) { return (p.M + 128 / nk - 1) / (128 / nk); };
+    // One pair of query tiles per workgroup while that fills every CU twice
+    // (512 workgroups), with as few key groups as do; else one query tile each,
+    // on two key groups if that is more than one workgroup per CU, else (D = 64)
+    // on four.  us at H = 32, with the cache pass: D = 64, M = 4096 pairs on one
+    // / two key groups 101 / 116; M = 2048 46 / 40; M = 1024 two key groups,
+    // pairs / single tiles 22.3 / 20.3; M = 512 single tiles, two / four key
+    // groups 13.5 / 12.5; D = 128, M = 1000 two key groups, pairs / single 29.8 / 27.6.
+    uint32_t nk = 1;
+    while (nk < 2 && (qtiles(nk) + 1) / 2 * p.H < 512) nk *= 2;
+    const int paired = (qtiles(nk) + 1) / 2 * p.H >= 512;
+    if (!paired && p.D == 64 && qtiles(2) * p.H <= 256) nk = 4;
+    switch (p.D + nk) {
+        case 65: return launch_attn<64, 1>(p, paired, st);
+        case 66: return launch_attn<64, 2>(p, paired, st);
+        case 68: return launch_attn<64, 4>(p, paired, st);
+        case 129: return launch_attn<128, 1>(p, paired, st);
+        default: return launch_attn<128, 2>(p, paired, st);
     }
 }
 

@@ -991,6 +991,27 @@ def test_flash_attention_gqa(bridge, oracle, H, Hkv, M, D):
     assert maxdiff(host(O), ref) <= TOL
 
 
+@pytest.mark.parametrize("H,Hkv,M,D", [(256, 2, 400, 64), (128, 1, 400, 64), (64, 2, 400, 64), (8, 8, 400, 64),
+                                       (256, 2, 330, 128), (128, 1, 390, 128), (16, 4, 390, 128), (2, 1, 65, 128)])
+def test_flash_attention_schedules(bridge, oracle, H, Hkv, M, D):
+    """Every split of the attention kernel: pairs of 128- and 64-query tiles
+    (512 workgroups or more; an odd tile count leaves a middle tile alone), single
+    64-query tiles on two key groups, 32-query tiles on four, with a last key tile
+    of 128 that runs past the 64-key padding (M = 400, 330 and 390), in both output
+    layouts, bit-identical to each other."""
+    rng = np.random.default_rng(H * M + D)
+    Q = (rng.standard_normal((H, M, D)) * 0.35).astype(np.float16)
+    K, V = ((rng.standard_normal((Hkv, M, D)) * 0.35).astype(np.float16) for _ in range(2))
+    Kq, Vq = oracle.quantize_q8_0(K), oracle.quantize_q8_0(V)
+    scale = float(np.float32(1.0) / np.sqrt(np.float32(D)))
+    O, Ot = empty16(H, M, D), empty16(M, H * D)
+    bridge.dispatch_flash_attn_q8_0_gqa(dev(Q), dev(Kq), dev(Vq), O, H, Hkv, M, D, scale)
+    bridge.dispatch_flash_attn_q8_0_gqa(dev(Q), dev(Kq), dev(Vq), Ot, H, Hkv, M, D, scale, o_token_major=True)
+    bridge.synchronize()
+    assert maxdiff(host(O), oracle.attention_q8_0_gqa(Q, Kq, Vq, Hkv, scale)) <= TOL
+    np.testing.assert_array_equal(host(Ot).reshape(M, H, D).transpose(1, 0, 2), host(O))
+
+
 @pytest.mark.parametrize("norm_type,rope,traditional,Hq,Hkv,D", [(1, True, False, 4, 2, 64), (2, True, True, 4, 4, 64),
                                                                   (1, False, False, 4, 1, 64),
                                                                   (1, True, False, 2, 1, 128)])
