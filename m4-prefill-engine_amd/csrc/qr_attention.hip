@@ -281,7 +281,7 @@ constexpr int kLmBytes = 2048;  // row sums and maxima of the merge
 __device__ __forceinline__ void attn_copy(uint32_t lds_addr, uint32_t voff, u4_t rsrc, uint32_t soff) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :: "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(rsrc),
-                    "s"(__builtin_amdgcn_readfirstlane(soff)));
+                    "s"(__builtin_amdgcn_readfirstlane(soff)) : "m0");
 }
 __device__ __forceinline__ u4_t attn_rsrc(const void* base, uint32_t bytes) {
     const uint64_t a = reinterpret_cast<uint64_t>(base);

@@ -69,7 +69,7 @@ __device__ __forceinline__ u4_t scalar_rsrc(const void* base, uint32_t bytes) {
 __device__ __forceinline__ void copy_lds(uint32_t lds_addr, uint32_t voff, u4_t rsrc, uint32_t soff) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :: "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(rsrc),
-                    "s"(__builtin_amdgcn_readfirstlane(soff)));
+                    "s"(__builtin_amdgcn_readfirstlane(soff)) : "m0");
 }
 
 // The packed bytes of one column for one round of 4 steps (128 K), as kUnits
