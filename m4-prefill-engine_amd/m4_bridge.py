@@ -135,6 +135,16 @@ def _is_torch(x: Any) -> bool:
     return type(x).__module__.startswith("torch")
 
 
+def _current_stream(device: int) -> int:
+    """Handle of torch's current stream on a device.  The raw getter returns it
+    without building a Stream object (0.2 instead of 2.0 us, of ~8 us that an
+    eager call takes on the host)."""
+    import torch
+
+    get = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return get(device) if get is not None else torch.cuda.current_stream(device).cuda_stream
+
+
 class HIPBridge:
     """Counterpart of the reference's MetalUMABridge (core/bridge/m4_bridge.py:47-242)."""
 
@@ -166,7 +176,7 @@ class HIPBridge:
             if not arr.is_contiguous():
                 arr = arr.contiguous()
                 cls._retained_contig.append(arr)
-            return int(arr.data_ptr()), int(arr.numel() * arr.element_size())
+            return arr.data_ptr(), arr.nbytes
         import numpy as np
 
         a = arr
@@ -182,9 +192,7 @@ class HIPBridge:
         the kernels are ordered after the work that produced the inputs."""
         for b in bufs:
             if _is_torch(b) and b.is_cuda:
-                import torch
-
-                self._lib.m4_bridge_set_stream(ctypes.c_void_p(torch.cuda.current_stream(b.device).cuda_stream))
+                self._lib.m4_bridge_set_stream(_current_stream(b.get_device()))
                 return
 
     def _check(self, name: str, ret: int) -> int:
