@@ -166,7 +166,7 @@ static WaveCost wave_cost(int shape, bool q4k) {
         case 0: return q4k ? WaveCost{68, 77} : WaveCost{51, 72};
         case 3: return q4k ? WaveCost{61, 77} : WaveCost{50, 72};
         case 1: return q4k ? WaveCost{39.5f, 47} : WaveCost{31, 39};
-        case 4: return q4k ? WaveCost{33, 36} : WaveCost{25, 32};
+        case 4: return q4k ? WaveCost{33, 34.5f} : WaveCost{25, 28};
         case 5: return q4k ? WaveCost{24, 29} : WaveCost{19, 26};
         case 6: return q4k ? WaveCost{27, 31} : WaveCost{18.5f, 25};
         case 7: return q4k ? WaveCost{97, 130} : WaveCost{81, 122};
@@ -180,14 +180,17 @@ static float plan_cost(const GemmParams& p, int shape, uint32_t ks) {
     float c = (float)(T / 256) * w.hi;
     if (rem) c += w.lo + (rem > 128 ? (w.hi - w.lo) * (float)(rem - 128) / 128.0f : 0.0f);
     c *= (float)p.K / (4096.0f * (float)ks);
-    // the partials' round trip (~4.5 TB/s) and the reduction kernel
-    if (ks > 1) c += 4.0f + (float)ks * (float)p.M * (float)columns_of(p) * (p.W2 ? 16.0f : 8.0f) / 4.5e6f;
+    // the reduction kernel (each split's loads in turn) and the partials' round trip at ~4.5 TB/s
+    if (ks > 1) c += 2.5f + 0.35f * (float)ks + (float)ks * (float)p.M * (float)columns_of(p) * (p.W2 ? 16.0f : 8.0f) / 4.5e6f;
     return c;
 }
 
-// The base shape with its K split, unless another shape without a split is
-// cheaper by its tile counts (so no call needs split-K partials that the base
-// choice would not).
+// The base shape with its K split, unless another is cheaper by its tile counts:
+// any shape without a split, or, where the base splits, 128- or 64-row tiles with
+// as many splits or fewer (so no call needs more split-K partials than the base
+// choice would).  MLX, M = 77, K = 8192, N = 2048: 16 splits of 128-row tiles
+// 20.8 us, 8 of 64-row tiles 16.4 (launch included); M = 128, K = N = 4096
+// 21.1 -> 16.3.
 void gemm_plan(GemmParams& p) {
     const bool dual = p.W2 != nullptr;
     p.shape = rb_pick(p.format, p.M, p.N, p.K, dual);
@@ -203,16 +206,30 @@ void gemm_plan(GemmParams& p) {
         const bool groups_ok = p.K % 128 == 0, wide = groups_ok && wide_format(p.format);
         const int cand[6] = {dual ? 2 : 1, dual ? -1 : (heavy ? 3 : 0), dual ? (wide ? 8 : -1) : (wide ? 7 : -1),
                              dual || !groups_ok ? -1 : 6, dual || !groups_ok || p.M > 128 ? -1 : 5, dual ? -1 : 4};
-        float best = 0.97f * plan_cost(p, p.shape, p.ksplit);
+        const float base = plan_cost(p, p.shape, p.ksplit);
+        const float margin = 0.08f * base;  // a near tie keeps the base's split (M = 640, K = 4096, N = 1024 ran even)
+        // one kernel without partials on a tie: M = 700, K = 4096, N = 1024 18.7 us, split 19.4
+        float best = p.ksplit > 1 ? base : 0.97f * base;
+        uint32_t ksplit = p.ksplit;
         for (int s : cand) {
             if (s < 0) continue;
             const float c = plan_cost(p, s, 1);
             if (c < best) {
                 best = c;
                 p.shape = s;
-                p.ksplit = 1;
+                ksplit = 1;
             }
         }
+        for (int s : {1, 4})
+            for (uint32_t ks = 2; !dual && ks <= p.ksplit; ks *= 2) {
+                const float c = plan_cost(p, s, ks) + margin;
+                if (c < best) {
+                    best = c;
+                    p.shape = s;
+                    ksplit = ks;
+                }
+            }
+        p.ksplit = ksplit;
     }
     p.group_m = (p.M + rb_dims(p.shape).bm - 1) / rb_dims(p.shape).bm >= 4 ? 4u : 2u;
 }

@@ -453,6 +453,36 @@ def test_few_rows(bridge, oracle, fmt, layout, M, K, N):
     tolerance.check(host(Y), gold, tolerance.gemm_bound(gold, absxw(oracle, fmt, X, W, K, N), K))
 
 
+@pytest.mark.parametrize("fmt", [0, 1, 2, 3, 8])
+@pytest.mark.parametrize("layout,M,K,N", [("plain", 77, 8192, 2046), ("residual", 128, 4096, 4096),
+                                          ("head", 256, 2048, 512), ("plain", 384, 4096, 1024),
+                                          ("plain", 65, 2048, 2048)])
+def test_split_k_plans(bridge, oracle, fmt, layout, M, K, N):
+    """Projections whose K split and tile height are chosen together (64-row
+    tiles with fewer splits than 128-row ones, a full and a ragged last row
+    tile, a ragged N), against the oracle on a row sample with every column."""
+    X = synth.activations(M, K, 190 + fmt, std=0.35)
+    W = weights("quantized", fmt, N, K, 191 + fmt)
+    rows = np.unique(np.r_[0, 31, 32, 63, 64, M - 1])
+    Xs = np.ascontiguousarray(X[rows])
+    Y = empty16(M, N)
+    R = None
+    if layout == "head":
+        bridge.dispatch_head_gemm(dev(X), dev(W), Y, fmt, M, N // 64, 64, K)
+    elif layout == "residual":
+        R = synth.activations(M, N, 192)
+        bridge.dispatch_gemm_residual(dev(X), dev(W), dev(R), Y, fmt, M, K, N)
+        R = np.ascontiguousarray(R[rows])
+    else:
+        bridge.dispatch_router_gemm(dev(X), dev(W), Y, fmt, M, K, N)
+    bridge.synchronize()
+    y = host(Y)
+    if layout == "head":
+        y = y.reshape(N // 64, M, 64).transpose(1, 0, 2).reshape(M, N)
+    gold = oracle.gemm(fmt, Xs, W, N, R=R)
+    tolerance.check(y[rows], gold, tolerance.gemm_bound(gold, absxw(oracle, fmt, Xs, W, K, N), K))
+
+
 @pytest.mark.parametrize("fmt", [0, 2])
 def test_wide_tiles_decode_bit_exact_mixed_exact_paths(bridge, oracle, fmt):
     """One-hot X through the 256 x 256 tiles with a third of the blocks outside
