@@ -275,6 +275,11 @@ __global__ void __launch_bounds__(256) kv_prep_kernel(const void* Ksrc, const vo
 constexpr int tile_keys(int D) { return D == 64 ? 128 : 64; }  // 32 KB of K and V^T per tile at either width
 constexpr int kTileBytes = 32768;
 constexpr int kLmBytes = 2048;  // row sums and maxima of the merge
+// Reference point of a row that has seen no score above -infinity: finite, so
+// that such scores weigh exp2(-inf - kNoScore) = 0 in every key group (from
+// -infinity it would be exp2(NaN), and one key group whose first keys all score
+// -infinity would make the whole row NaN).
+constexpr float kNoScore = -3.402823466e38f;
 
 // 1 KB global -> LDS copy (16 bytes per lane, lane l to lds_addr + 16 l); not
 // known to the compiler, so every reader waits for it explicitly.
@@ -381,14 +386,14 @@ __global__ void __launch_bounds__(256, 2) flash_attn_kernel(AttnParams p, int pa
             qf[kk] = __builtin_bit_cast(h8_t, ld_b128(qr_, off));
             if (neg) qf[kk] = -qf[kk];
         }
-        m_run = -INFINITY;
+        m_run = kNoScore;
         l_run = 0.0f;
 #pragma unroll
         for (int t = 0; t < DT; t++) o[t] = f16v_t{};
     };
     auto store = [&]() {
         const float l = l_run + __shfl_xor(l_run, 32);
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        const float inv = 1.0f / l;
         const int my_q = qw + j;
         if (my_q >= M) return;
 #pragma unroll
@@ -504,8 +509,7 @@ __global__ void __launch_bounds__(256, 2) flash_attn_kernel(AttnParams p, int pa
                 const float* x = reinterpret_cast<const float*>(buf) + sl * (DT * 16 * 64);
                 const f2_t q = *reinterpret_cast<const f2_t*>(lm + (sl * 64 + lane) * 2);
                 const float m = fmaxf(q.y, m_run);
-                const float fa = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(q.y - m);
-                const float fb = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m);
+                const float fa = __builtin_amdgcn_exp2f(q.y - m), fb = __builtin_amdgcn_exp2f(m_run - m);
 #pragma unroll
                 for (int t = 0; t < DT; t++)
 #pragma unroll

@@ -1042,6 +1042,31 @@ def test_flash_attention_schedules(bridge, oracle, H, Hkv, M, D):
     np.testing.assert_array_equal(host(Ot).reshape(M, H, D).transpose(1, 0, 2), host(O))
 
 
+@pytest.mark.parametrize("H,Hkv,M,D", [(256, 2, 400, 64), (128, 1, 400, 64), (64, 2, 400, 64), (8, 8, 400, 64),
+                                       (256, 2, 330, 128), (128, 1, 390, 128), (16, 4, 390, 128)])
+def test_flash_attention_keys_scored_minus_infinity(bridge, oracle, H, Hkv, M, D):
+    """Keys 32..127 score -infinity for every query (a K block whose scale
+    overflows binary16 times its code): they weigh nothing, also where they are
+    all that a key group sees first, in every split of the kernel."""
+    rng = np.random.default_rng(H + M + D)
+    Q = (rng.standard_normal((H, M, D)) * 0.35).astype(np.float16)
+    Q[:, :, 0] = np.abs(Q[:, :, 0]) + np.float16(0.25)
+    K, V = ((rng.standard_normal((Hkv, M, D)) * 0.35).astype(np.float16) for _ in range(2))
+    Kq, Vq = oracle.quantize_q8_0(K), oracle.quantize_q8_0(V)
+    blk = Kq.reshape(Hkv, M, D // 32, 34)[:, 32:128, 0]
+    blk[...] = 0
+    blk[..., :2] = np.frombuffer(np.float16(1000.0).tobytes(), np.uint8)
+    blk[..., 2] = 256 - 127  # code -127: half(-127 * 1000) = -inf in d = 0, zeros beside it
+    assert np.isneginf(oracle.dequantize_q8_0(Kq).reshape(Hkv, M, D)[:, 32:128, 0]).all()
+    scale = float(np.float32(1.0) / np.sqrt(np.float32(D)))
+    O = empty16(H, M, D)
+    bridge.dispatch_flash_attn_q8_0_gqa(dev(Q), dev(Kq), dev(Vq), O, H, Hkv, M, D, scale)
+    bridge.synchronize()
+    ref = oracle.attention_q8_0_gqa(Q, Kq, Vq, Hkv, scale)
+    assert np.isfinite(ref).all()
+    assert maxdiff(host(O), ref) <= TOL
+
+
 @pytest.mark.parametrize("norm_type,rope,traditional,Hq,Hkv,D", [(1, True, False, 4, 2, 64), (2, True, True, 4, 4, 64),
                                                                   (1, False, False, 4, 1, 64),
                                                                   (1, True, False, 2, 1, 128)])
