@@ -220,6 +220,21 @@ M4_API int m4_bridge_dequantize(void* W_ptr, size_t W_bytes, void* out_ptr, size
 M4_API int m4_bridge_dispatch_gemm_noalloc(void* X_ptr, size_t X_bytes, void* W_ptr, size_t W_bytes, void* Y_ptr,
                                            size_t Y_bytes, int format, uint32_t M, uint32_t K, uint32_t N);
 
+/* No counterpart in the reference: which kernel a projection of [M, K]
+ * activations runs here, from the same choice that the dispatches make (host
+ * arithmetic only, no GPU and no initialization needed).  N holds the widths of
+ * `groups` projections launched together (1, or 3 for a layer's Q, K and V);
+ * `swiglu`: the fused gate and up projection.  0, -2 (null), -3 (format), -4. */
+enum { M4_KERNEL_FEW_ROWS = 0, M4_KERNEL_SMALL_M = 1, M4_KERNEL_TILED = 2, M4_KERNEL_WIDE = 3 };
+typedef struct {
+    int kernel;                   /* M4_KERNEL_* */
+    uint32_t tile_rows, tile_cols; /* outputs of one workgroup */
+    uint32_t k_groups;            /* K groups inside a workgroup */
+    uint32_t k_splits;            /* K splits over workgroups (> 1: a reduction kernel follows) */
+} m4_projection_plan_t;
+M4_API int m4_bridge_projection_plan(int format, uint32_t M, uint32_t K, const uint32_t* N, uint32_t groups, int swiglu,
+                                     m4_projection_plan_t* plan);
+
 /* Run subsequent work on `stream` (a hipStream_t, e.g. torch's current
  * stream); NULL restores the bridge's own stream.  Returns 0 or -1. */
 M4_API int m4_bridge_set_stream(void* stream);

@@ -299,7 +299,8 @@ int launch_ws(const qr::GemmParams& p0, float* fixed_ws, size_t fixed_floats) {
         *ws = g_sk_ws;
         return 0;
     };
-    if (qr::gemv_fits(p)) {
+    const qr::Route route = qr::choose_route(p);
+    if (route == qr::Route::kFewRows) {
         hipError_t e = qr::launch_gemv(p, g_stream);
         if (e != hipSuccess) {
             set_error("launch_gemv", e);
@@ -307,7 +308,7 @@ int launch_ws(const qr::GemmParams& p0, float* fixed_ws, size_t fixed_floats) {
         }
         return 0;
     }
-    if (p.ngroups <= 1 && qr::skinny_supported(p)) {
+    if (route == qr::Route::kSmallM) {
         const size_t floats = qr::skinny_workspace_floats(p.M, p.N, p.K);
         float* ws = nullptr;
         if (int rc = workspace(floats ? floats : 1, &ws)) return rc;
@@ -318,7 +319,6 @@ int launch_ws(const qr::GemmParams& p0, float* fixed_ws, size_t fixed_floats) {
         }
         return 0;
     }
-    qr::gemm_plan(p);
     if (p.ksplit > 1) {
         if (int rc = workspace(qr::gemm_workspace_floats(p), &p.ws)) return rc;
     }
@@ -447,6 +447,36 @@ int m4_bridge_dispatch_gemm_noalloc(void* X, size_t Xb, void* W, size_t Wb, void
     p.M = M; p.N = N; p.K = K;
     p.col_bytes = wbytes / N;
     return launch_ws(p, ws, kScratchFloats);
+}
+
+int m4_bridge_projection_plan(int format, uint32_t M, uint32_t K, const uint32_t* N, uint32_t groups, int swiglu,
+                              m4_projection_plan_t* plan) {
+    if (!N || !plan) return -2;
+    if (!has_kernels(format)) return -3;
+    if (M == 0 || K == 0 || K % qr::get_quant_info(static_cast<qr::QuantFormat>(format)).block_size || groups == 0 ||
+        groups > 3 || (swiglu && groups > 1))
+        return -4;
+    for (uint32_t g = 0; g < groups; g++)
+        if (N[g] == 0) return -4;
+    qr::GemmParams p{};
+    p.format = format;
+    p.M = M; p.N = N[0]; p.K = K;
+    p.col_bytes = qr::kernel_weight_bytes(format, K, 1);
+    static const uint8_t other = 0;  // the plan only asks whether there is a second matrix
+    p.W2 = swiglu ? &other : nullptr;
+    p.ngroups = groups;
+    for (uint32_t g = 1; g < groups; g++) p.Nx[g - 1] = N[g];
+    switch (qr::choose_route(p)) {
+        case qr::Route::kFewRows: *plan = {M4_KERNEL_FEW_ROWS, 16, qr::gemv_tile_columns(p), 1, 1}; break;
+        case qr::Route::kSmallM:
+            *plan = {M4_KERNEL_SMALL_M, (M + 15) / 16 * 16, qr::skinny_tile_columns(p), 1, qr::skinny_ksplit(p)};
+            break;
+        case qr::Route::kTiled: {
+            const qr::TileInfo t = qr::gemm_tile(p);
+            *plan = {t.rows == 256 ? M4_KERNEL_WIDE : M4_KERNEL_TILED, t.rows, t.cols, t.k_groups, p.ksplit};
+        }
+    }
+    return 0;
 }
 
 int m4_bridge_dispatch_router_gemm(void* X, size_t Xb, void* W, size_t Wb, void* Y, size_t Yb, int format,

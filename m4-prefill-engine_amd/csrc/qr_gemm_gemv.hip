@@ -215,6 +215,13 @@ __global__ void __launch_bounds__(gemv::kThreads, (gemv::waves_per_simd<F, NC * 
     }
 }
 
+// Column tiles of p, all groups.
+static uint32_t column_tiles(const GemmParams& p, uint32_t cw) {
+    uint32_t t = (p.N + cw - 1) / cw;
+    for (uint32_t g = 1; g < p.ngroups && g < 3; g++) t += (p.Nx[g - 1] + cw - 1) / cw;
+    return t;
+}
+
 // Where this kernel is the fastest (each launch in a graph, us, other kernel ->
 // this one):
 //  * SwiGLU: always, against the 128-row tiles (MLX, K = 4096, N = 14336:
@@ -237,19 +244,17 @@ bool gemv_fits(const GemmParams& p) {
     return tiles <= 1024 && (p.M <= 8 || tiles <= 128);
 }
 
+// Two column tiles per workgroup when the workgroups of one would not be
+// resident at once (MLX N = 14336, K = 4096, M = 1: 15.5 -> 12.8 us).
+uint32_t gemv_tile_columns(const GemmParams& p) { return !p.W2 && column_tiles(p, 16) > 512 ? 32 : 16; }
+
 template <int F>
 static hipError_t launch_gemv_f(const GemmParams& p, hipStream_t st) {
-    // two column tiles per workgroup when the workgroups of one would not be
-    // resident at once (MLX N = 14336, K = 4096, M = 1: 15.5 -> 12.8 us)
-    auto tiles = [&](uint32_t cw) {
-        uint32_t t = (p.N + cw - 1) / cw;
-        for (uint32_t g = 1; g < p.ngroups && g < 3; g++) t += (p.Nx[g - 1] + cw - 1) / cw;
-        return t;
-    };
-    const dim3 block(gemv::kThreads);
-    if (p.W2) hipLaunchKernelGGL((gemv_kernel<F, 1, 2>), dim3(tiles(16)), block, 0, st, p);
-    else if (tiles(16) > 512) hipLaunchKernelGGL((gemv_kernel<F, 2, 1>), dim3(tiles(32)), block, 0, st, p);
-    else hipLaunchKernelGGL((gemv_kernel<F, 1, 1>), dim3(tiles(16)), block, 0, st, p);
+    const uint32_t cw = gemv_tile_columns(p);
+    const dim3 grid(column_tiles(p, cw)), block(gemv::kThreads);
+    if (p.W2) hipLaunchKernelGGL((gemv_kernel<F, 1, 2>), grid, block, 0, st, p);
+    else if (cw == 32) hipLaunchKernelGGL((gemv_kernel<F, 2, 1>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((gemv_kernel<F, 1, 1>), grid, block, 0, st, p);
     return hipGetLastError();
 }
 

@@ -234,6 +234,18 @@ void gemm_plan(GemmParams& p) {
     p.group_m = (p.M + rb_dims(p.shape).bm - 1) / rb_dims(p.shape).bm >= 4 ? 4u : 2u;
 }
 
+Route choose_route(GemmParams& p) {
+    if (gemv_fits(p)) return Route::kFewRows;
+    if (p.ngroups <= 1 && skinny_supported(p)) return Route::kSmallM;
+    gemm_plan(p);
+    return Route::kTiled;
+}
+
+TileInfo gemm_tile(const GemmParams& p) {
+    const RbShape d = rb_dims(p.shape);
+    return {d.bm, d.bn, p.shape == 5 || p.shape == 6 ? 2u : 1u};
+}
+
 size_t gemm_workspace_floats(const GemmParams& p) {
     return p.ksplit > 1 ? (size_t)p.ksplit * p.M * columns_of(p) * (p.W2 != nullptr ? 2 : 1) : 0;
 }

@@ -721,6 +721,14 @@ bool skinny_supported(const GemmParams& p) {
 
 bool skinny_one_kernel(const GemmParams& p) { return st_plan(p.format, p.M, p.N, p.K); }
 
+uint32_t skinny_tile_columns(const GemmParams& p) { return skinny_one_kernel(p) ? 16 : kSkCols; }
+
+uint32_t skinny_ksplit(const GemmParams& p) {
+    uint32_t ks = 1, gpw;
+    if (!skinny_one_kernel(p)) sk_plan(p.format, p.M, p.N, p.K, &ks, &gpw);
+    return ks;
+}
+
 hipError_t launch_gemm_skinny(const GemmParams& p, float* ws, hipStream_t st) {
     switch (p.format) {
         case QUANT_Q4_0: return launch_sk_m<QUANT_Q4_0>(p, ws, st);

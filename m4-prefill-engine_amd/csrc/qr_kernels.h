@@ -45,6 +45,7 @@ hipError_t launch_splitk_reduce(const float* ws, uint32_t ks, uint32_t M, uint32
 // One-kernel projection or SwiGLU for M <= 16 (no workspace), and whether it
 // takes p.
 bool gemv_fits(const GemmParams& p);
+uint32_t gemv_tile_columns(const GemmParams& p);
 hipError_t launch_gemv(const GemmParams& p, hipStream_t st);
 
 // Small-M weight-streaming projection (M <= 64, no SwiGLU).  `ws` holds
@@ -53,8 +54,18 @@ hipError_t launch_gemv(const GemmParams& p, hipStream_t st);
 bool skinny_supported(const GemmParams& p);
 // Whether launch_gemm_skinny runs p as one kernel, without a K split.
 bool skinny_one_kernel(const GemmParams& p);
+uint32_t skinny_tile_columns(const GemmParams& p);
+uint32_t skinny_ksplit(const GemmParams& p);
 size_t skinny_workspace_floats(uint32_t M, uint32_t N, uint32_t K);
 hipError_t launch_gemm_skinny(const GemmParams& p, float* ws, hipStream_t st);
+// The kernel that runs p; plans it (gemm_plan) when that is the tiled one.
+enum class Route { kFewRows, kSmallM, kTiled };
+Route choose_route(GemmParams& p);
+// Outputs of one workgroup of the planned shape, and its K groups.
+struct TileInfo {
+    uint32_t rows, cols, k_groups;
+};
+TileInfo gemm_tile(const GemmParams& p);
 hipError_t launch_dequant(int format, const uint8_t* W, _Float16* out, uint32_t K, uint32_t N, size_t col_bytes,
                           hipStream_t st);
 

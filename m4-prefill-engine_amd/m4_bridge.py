@@ -67,6 +67,7 @@ SIGNATURES = {
     "m4_bridge_shutdown": ([], None),
     "m4_bridge_validate_gemm": ([_VP, _SZ, _VP, _SZ, _VP, _SZ, _I, _U32, _U32, _U32], _I),
     "m4_bridge_dispatch_gemm_noalloc": ([_VP, _SZ, _VP, _SZ, _VP, _SZ, _I, _U32, _U32, _U32], _I),
+    "m4_bridge_projection_plan": ([_I, _U32, _U32, ctypes.POINTER(_U32), _U32, _I, _VP], _I),
     "m4_bridge_dispatch_router_gemm": ([_VP, _SZ, _VP, _SZ, _VP, _SZ, _I, _U32, _U32, _U32], _I),
     "m4_bridge_dispatch_head_gemm": ([_VP, _SZ, _VP, _SZ, _VP, _SZ, _I, _U32, _U32, _U32, _U32], _I),
     "m4_bridge_dispatch_router_kernel": ([ctypes.c_char_p, _VP, _SZ, _VP, _SZ, _VP, _SZ,
@@ -112,6 +113,32 @@ class CodecInfo(ctypes.Structure):
         ("gemm_kernel_name", ctypes.c_char_p),
         ("head_gemm_kernel_name", ctypes.c_char_p),
     ]
+
+
+class ProjectionPlan(ctypes.Structure):
+    """m4_projection_plan_t (include/m4_mlx_bridge.h)."""
+    _fields_ = [("kernel", ctypes.c_int), ("tile_rows", _U32), ("tile_cols", _U32), ("k_groups", _U32),
+                ("k_splits", _U32)]
+
+    KERNELS = ("few_rows", "small_m", "tiled", "wide")
+
+    @property
+    def kernel_name(self) -> str:
+        return self.KERNELS[self.kernel]
+
+    def astuple(self) -> tuple:
+        return (self.kernel_name, self.tile_rows, self.tile_cols, self.k_groups, self.k_splits)
+
+
+def projection_plan(lib: ctypes.CDLL, format_id: int, M: int, K: int, *N: int, swiglu: bool = False) -> ProjectionPlan:
+    """The kernel that [M, K] x [N, K]^T in a format runs (several N: projections
+    launched together), from the library's own choice; no GPU needed."""
+    plan = ProjectionPlan()
+    rc = lib.m4_bridge_projection_plan(int(format_id), M, K, (_U32 * len(N))(*N), len(N), int(swiglu),
+                                       ctypes.byref(plan))
+    if rc:
+        raise ValueError(f"m4_bridge_projection_plan failed with status code {rc}")
+    return plan
 
 
 def load_library(path: Optional[Union[str, Path]] = None) -> ctypes.CDLL:

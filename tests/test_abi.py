@@ -220,3 +220,36 @@ def test_extract_buffer_strided_and_offset_views(libpath):
         assert sub - base == 10 * 64 * 2 and sub_bytes == 10 * 64 * 2
     assert len(B._retained_contig) >= 2
     B._retained_contig.clear()
+
+
+def test_projection_plan(lib):
+    """The kernel choice as host arithmetic: refusals, and what must hold for any
+    plan (a split divides K into whole 256-element super-blocks of at least 512; the
+    kernels with K groups and the 256-row tiles take K whole)."""
+    import ctypes
+
+    n = (ctypes.c_uint32 * 3)(4096, 1024, 1024)
+    out = m4_bridge.ProjectionPlan()
+    call = lib.m4_bridge_projection_plan
+    assert call(0, 1, 4096, None, 1, 0, ctypes.byref(out)) == -2
+    assert call(0, 1, 4096, n, 1, 0, None) == -2
+    assert call(9, 1, 4096, n, 1, 0, ctypes.byref(out)) == -3
+    for args in ((0, 0, 4096, n, 1, 0), (0, 1, 0, n, 1, 0), (2, 1, 4128, n, 1, 0), (0, 1, 4096, n, 0, 0),
+                 (0, 1, 4096, n, 4, 0), (0, 1, 4096, n, 3, 1), (0, 1, 4096, (ctypes.c_uint32 * 1)(0), 1, 0)):
+        assert call(*args, ctypes.byref(out)) == -4, args
+    for fmt in range(9):
+        for K in (256, 1024, 2048, 4096, 11008, 14336):
+            for M in (1, 2, 8, 16, 17, 33, 64, 65, 128, 129, 200, 256, 1000, 2048, 8192):
+                for N in (64, 1000, 4096, 14336, 28672):
+                    for kind in ("plain", "swiglu", "grouped"):
+                        ns = (N, 64, 256) if kind == "grouped" else (N,)
+                        p = m4_bridge.projection_plan(lib, fmt, M, K, *ns, swiglu=kind == "swiglu")
+                        t = (fmt, M, K, N, kind, p.astuple())
+                        assert p.k_splits >= 1 and K % (256 * p.k_splits) == 0, t
+                        if p.kernel_name == "few_rows":
+                            assert M <= 16 and p.k_splits == 1, t
+                        if p.kernel_name == "wide":
+                            assert p.k_splits == 1 and p.tile_rows == 256 and K % 128 == 0 and fmt in (0, 1, 2, 3, 8), t
+                        if p.kernel_name == "tiled":
+                            assert p.k_splits == 1 or K // p.k_splits >= 512, t
+                            assert p.k_groups == 1 or (p.k_splits == 1 and K % 128 == 0), t

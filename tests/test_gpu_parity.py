@@ -45,6 +45,13 @@ def absxw(oracle, fmt, X, W, K, N):
     return np.abs(X.astype(np.float64)) @ np.abs(oracle.dequantize_f64(fmt, W, K, N)).T
 
 
+def plan(bridge, fmt, M, K, *N, swiglu=False):
+    """(kernel, tile rows, tile columns, K groups, K splits) that the library runs a projection with."""
+    import m4_bridge
+
+    return m4_bridge.projection_plan(bridge.lib, fmt, M, K, *N, swiglu=swiglu).astuple()
+
+
 def weights(kind, fmt, N, K, seed):
     return synth.random_blocks(fmt, N, K, seed) if kind == "random" else synth.quantized_weights(fmt, N, K, seed)
 
@@ -380,16 +387,20 @@ def test_gemm_decode_bit_exact_mixed_exact_paths(bridge, oracle, fmt, M, K, N):
 
 
 @pytest.mark.parametrize("fmt", [0, 1, 2, 3, 8])
-@pytest.mark.parametrize("layout,M,K,N", [("plain", 500, 128, 22038), ("plain", 513, 256, 22040), ("head", 500, 384, 22016),
-                                          ("residual", 511, 640, 22016), ("swiglu", 500, 128, 9000),
-                                          ("swiglu", 512, 384, 9002)])
-def test_wide_tiles(bridge, oracle, fmt, layout, M, K, N):
+@pytest.mark.parametrize("layout,M,K,N,kernel", [("plain", 500, 128, 22038, "wide"), ("plain", 513, 256, 22040, "tiled"),
+                                                 ("plain", 513, 256, 21752, "wide"), ("head", 500, 384, 22016, "wide"),
+                                                 ("residual", 511, 640, 22016, "wide"), ("swiglu", 500, 128, 9000, "wide"),
+                                                 ("swiglu", 512, 384, 9002, "wide")])
+def test_wide_tiles(bridge, oracle, fmt, layout, M, K, N, kernel):
     """The 256 x 256 tiles (more than one wave of 128 x 256 tiles): ragged M
-    and N (an N that is no multiple of 8, whose stores are per element), K of
+    and N (an N that is no multiple of 8, whose stores are per element, and one
+    that is), a last row tile of one row (its second wave row empty), K of
     one round of 4 steps (128), two, three and five (the rings of three X
     pairs and two weight slots wrap at every phase), each output layout and
-    SwiGLU, against the oracle on a row sample with every column."""
+    SwiGLU, against the oracle on a row sample with every column.  Three row tiles
+    of 87 columns are more than one wave: there the 128-row tiles are cheaper."""
     K = 256 * -(-K // 256) if fmt == 2 else K  # Q4_K: whole super-blocks
+    assert plan(bridge, fmt, M, K, N, swiglu=layout == "swiglu")[0] == kernel
     X = synth.activations(M, K, 170 + fmt, std=0.35)
     W = weights("quantized", fmt, N, K, 171 + fmt)
     rows = np.unique(np.r_[0, 1, 31, 32, 127, 128, 255, 256, M - 1])
@@ -425,6 +436,7 @@ def test_few_rows(bridge, oracle, fmt, layout, M, K, N):
     the eight waves idle), two and nine (waves with one and two), ragged N, two
     column tiles per workgroup (N = 14344: an odd tile count's last half
     empty), every layout and SwiGLU, every format, on every element."""
+    assert plan(bridge, fmt, M, K, N, swiglu=layout == "swiglu")[:3] == ("few_rows", 16, 32 if N > 8192 else 16)
     X = synth.activations(M, K, 180 + fmt, std=0.35)
     kind = "random" if fmt > 3 and fmt != 8 else "quantized"
     W = weights(kind, fmt, N, K, 181 + fmt)
@@ -1115,6 +1127,32 @@ def test_prefill_layer_short_prompts(bridge, oracle, fmt, M):
     # fp16 intermediates on both sides: an upstream tie moves an output by about
     # one step, whose size follows the largest value
     assert maxdiff(host(out), ref) <= 2 * max(TOL, float(tolerance.ulp16(np.abs(ref).max())))
+
+
+@pytest.mark.parametrize("fmt,M,Hq,Hkv,D,kernel", [(0, 1, 64, 2, 128, "few_rows"), (3, 5, 64, 2, 128, "few_rows"),
+                                                    (8, 16, 66, 33, 64, "few_rows"), (0, 4001, 15, 3, 128, "wide"),
+                                                    (1, 4001, 15, 3, 128, "wide"), (2, 4001, 18, 3, 128, "wide"),
+                                                    (3, 4001, 15, 3, 128, "wide"), (8, 4001, 15, 3, 128, "wide")])
+def test_prefill_layer_grouped_kernels(bridge, oracle, fmt, M, Hq, Hkv, D, kernel):
+    """Q, K and V of unequal widths as one launch of the few-row kernel with two
+    column tiles per workgroup (more than 512 tiles; 66 and 33 heads of 64: 132 and
+    66 pairs of tiles), and of the 256 x 256 tiles (widths of 7.5 and 1.5 tiles, Q4_K
+    of 9 and 1.5; a last row tile ragged), on a row sample of the layer's output."""
+    dm = Nm = 256 if fmt == 2 or kernel == "wide" else 512
+    got = plan(bridge, fmt, M, dm, Hq * D, Hkv * D, Hkv * D)
+    assert got[:3] == (kernel, 16, 32) if kernel == "few_rows" else got[:3] == (kernel, 256, 256), got
+    X = synth.activations(M, dm, 291)
+    shapes = [(Hq * D, dm), (Hkv * D, dm), (Hkv * D, dm), (dm, Hq * D), (Nm, dm), (Nm, dm), (dm, Nm)]
+    Ws = [weights("quantized", fmt, n, k, 292 + i) for i, (n, k) in enumerate(shapes)]
+    out = empty16(M, dm)
+    bridge.prefill_layer_ex(dev(X), None, *[dev(x) for x in Ws[:4]], None, *[dev(x) for x in Ws[4:]], out, fmt, M, dm,
+                            Hq, Hkv, D, Nm, D ** -0.5, rope=True, rope_theta=10000.0, rope_offset=3)
+    bridge.synchronize()
+    rows = np.unique(np.r_[0, 1, 127, 128, 255, 256, M // 2, M - 1])
+    rows = rows[rows < M]
+    ref = oracle.layer_ex_rows(fmt, X, None, *Ws[:4], None, *Ws[4:], rows, Hq, Hkv, D, Nm, D ** -0.5, rope=True,
+                               theta=10000.0, offset=3)
+    assert maxdiff(host(out)[rows], ref) <= 2 * max(TOL, float(tolerance.ulp16(np.abs(ref).max())))
 
 
 @pytest.mark.parametrize("fmt", [0, 1, 2, 3])
