@@ -150,86 +150,126 @@ static uint32_t columns_of(const GemmParams& p) {
     return n;
 }
 
-// One workgroup fits a CU, so a grid runs in waves of 256 tiles.  What a wave
-// takes, in us at K = 4096 (it is proportional to K but for ~5 us), per shape:
-// `lo` while at most half of the CUs have a tile, rising to `hi` when all have
-// (the clock falls as the chip fills).  Measured on MLX and Q4_0 weights (they
-// agree to 5%; ternary is ~10% faster at every shape) and on Q4_K, whose decode
-// is the heaviest; e.g. MLX at N = 14336: M = 900 128 x 128 tiles 142.7,
-// 128 x 256 121.2, 256 x 256 107.4; M = 450 71.4 / 61.6 / 82.4; M = 256
-// 37.0 / 52.5 / 81.5.
-struct WaveCost {
-    float lo, hi;
+// ---- the price of a plan ----
+// One workgroup fits a CU, so a grid runs in waves of 256 tiles.  A wave takes
+// `fix` us whatever K is (ramp, first loads, epilogue) and, per 4096 of K, `full`
+// us when every CU has a tile and `half` when at most half of them have (the
+// clock falls as the chip fills; for 64-row tiles the step from `half` to `full`
+// starts at an empty chip, else at half).  A K split adds its reduction kernel: r0
+// us, r1 per split and rb times the partials' round trip at 4.5 TB/s.
+// Least-squares fits to the times of every choice in graphs, weights rotated over
+// 300 MB: ~460 shapes per format, M 17 .. 4900, K 1024 .. 14336, N 256 .. 28672
+// (relative error 5 - 8% rms: 3 - 4% for the 256-row tiles, 8 - 10% for the 64-row
+// ones), less what all choices share (streaming X, W and Y).
+// Each format has its own: the decode, the bytes and how they are fetched move the
+// tiles against each other (M = 128, K = 4096, N = 14336, 128 x 64 against 64 x 128
+// with two K groups: g64 26.9 / 30.9 us, MLX 26.7 / 27.9, ternary 21.9 / 20.9, Q8_0
+// 34.8 / 42.7).
+struct TileCost {
+    float fix, full, half;
 };
-static WaveCost wave_cost(int shape, bool q4k) {
-    switch (shape) {
-        case 0: return q4k ? WaveCost{68, 77} : WaveCost{51, 72};
-        case 3: return q4k ? WaveCost{61, 77} : WaveCost{50, 72};
-        case 1: return q4k ? WaveCost{39.5f, 47} : WaveCost{31, 39};
-        case 4: return q4k ? WaveCost{33, 34.5f} : WaveCost{25, 28};
-        case 5: return q4k ? WaveCost{24, 29} : WaveCost{19, 26};
-        case 6: return q4k ? WaveCost{27, 31} : WaveCost{18.5f, 25};
-        case 7: return q4k ? WaveCost{97, 130} : WaveCost{81, 122};
-        case 8: return q4k ? WaveCost{94, 130} : WaveCost{79, 122};
-        default: return q4k ? WaveCost{66, 82} : WaveCost{53, 72};  // 2: SwiGLU 128 x 128
+struct FormatCost {
+    TileCost mid, big;          // 128 x 128; 128 x 256 (shape 0, or 3 for Q4_K and ternary)
+    TileCost low, low_split;    // 64 x 128 without and with a K split (other kernel instances)
+    TileCost kg, low_kg;        // 128 x 64 and 64 x 128 as two K groups
+    TileCost wide;              // 256 x 256
+    TileCost dual, dual_wide;   // SwiGLU: 128 x 128 and 256 x 128 outputs
+    float r0, r1, rb;           // reduction of a projection
+    float d0, d1, db;           // reduction of SwiGLU
+};
+static const FormatCost& format_cost(int f) {
+    static const FormatCost q4_0 = {{4.8f, 31.7f, 24.7f}, {7, 59.5f, 43.1f}, {3.2f, 22.7f, 18.5f}, {2.9f, 19.8f, 20},
+                                    {5.7f, 14.3f, 11.7f}, {3.4f, 21.3f, 16.8f}, {12.7f, 103.3f, 71.7f},
+                                    {4.5f, 55.3f, 45.5f}, {8.2f, 96, 76.5f}, 2.6f, 0.25f, 0.97f, 3.35f, 0.4f, 0.71f};
+    static const FormatCost mlx = {{4.8f, 32.5f, 23.9f}, {6.9f, 57.9f, 42.5f}, {2.5f, 21.1f, 18.6f}, {2.5f, 19.4f, 18.7f},
+                                   {6, 13, 11.6f}, {4.9f, 15.8f, 12.4f}, {12.1f, 103, 68.1f},
+                                   {5.3f, 52.1f, 44.7f}, {7.9f, 96.4f, 71.2f}, 2.8f, 0.25f, 0.94f, 3, 0.27f, 0.71f};
+    static const FormatCost q4_k = {{4.5f, 39.8f, 34.6f}, {5.7f, 71.1f, 54.4f}, {3.2f, 29.1f, 29}, {2.7f, 28.8f, 27.9f},
+                                    {5.3f, 19.6f, 18.2f}, {4.2f, 23.5f, 22}, {12.3f, 109.9f, 82.8f},
+                                    {5, 68.6f, 60}, {8.5f, 105.6f, 85.6f}, 3.85f, 0.15f, 0.55f, 4.1f, 0.31f, 0.73f};
+    static const FormatCost ternary = {{5.1f, 29.2f, 24.3f}, {6.7f, 51.6f, 38.4f}, {4, 15.8f, 16.6f}, {2.8f, 15.9f, 15.8f},
+                                       {5.5f, 12.8f, 12.2f}, {4.3f, 15.3f, 13.1f}, {12, 89, 67.3f},
+                                       {5.4f, 47.9f, 40.6f}, {8.4f, 84.1f, 69.7f}, 3.85f, 0.19f, 0.47f, 3, 0.31f, 0.85f};
+    static const FormatCost q8_0 = {{3.2f, 38.4f, 31.4f}, {5.2f, 69.9f, 60.6f}, {1.8f, 29.2f, 27.1f}, {1.8f, 25.6f, 26.4f},
+                                    {3.8f, 16.6f, 17.3f}, {1.8f, 29.8f, 27.2f}, {},
+                                    {3.1f, 52.1f, 59.3f}, {}, 3.35f, 0.3f, 1.1f, 3.95f, 0.41f, 0.85f};
+    static const FormatCost prism = {{4.4f, 32.2f, 26.4f}, {6.7f, 58.9f, 44.6f}, {3.3f, 21.1f, 20}, {2.8f, 21.3f, 19.7f},
+                                     {4.5f, 14.9f, 13.5f}, {3.8f, 18.1f, 15.7f}, {},
+                                     {4.9f, 47.1f, 44.6f}, {}, 2.9f, 0.27f, 1.2f, 3.35f, 0.41f, 1};
+    static const FormatCost g64 = {{5, 31.6f, 24.1f}, {6.7f, 59.4f, 43.2f}, {3, 20.5f, 18.5f}, {2.9f, 18.5f, 17.9f},
+                                   {5.2f, 13.4f, 13.2f}, {3.7f, 20, 17}, {12.3f, 102.8f, 68.7f},
+                                   {4.4f, 56.5f, 44.6f}, {8.2f, 95.9f, 72.3f}, 3.05f, 0.2f, 0.87f, 3.15f, 0.31f, 1};
+    switch (f) {
+        case QUANT_MLX_4BIT: return mlx;
+        case QUANT_Q4_K: return q4_k;
+        case QUANT_TERNARY_1_58: return ternary;
+        case QUANT_Q8_0: return q8_0;
+        case QUANT_PRISM_Q2_0: return prism;
+        case QUANT_MLX_4BIT_G64: return g64;
+        default: return q4_0;
     }
 }
 static float plan_cost(const GemmParams& p, int shape, uint32_t ks) {
-    const WaveCost w = wave_cost(shape, p.format == QUANT_Q4_K);
+    const FormatCost& f = format_cost(p.format);
+    const bool low = shape == 4 || shape == 6;
+    const TileCost& w = shape == 1 ? f.mid : shape == 0 || shape == 3 ? f.big : shape == 4 ? (ks > 1 ? f.low_split : f.low)
+                      : shape == 5 ? f.kg : shape == 6 ? f.low_kg : shape == 7 ? f.wide : shape == 8 ? f.dual_wide : f.dual;
     const uint32_t T = tiles_of(p, rb_dims(shape)) * ks, rem = T % 256;
-    float c = (float)(T / 256) * w.hi;
-    if (rem) c += w.lo + (rem > 128 ? (w.hi - w.lo) * (float)(rem - 128) / 128.0f : 0.0f);
-    c *= (float)p.K / (4096.0f * (float)ks);
-    // the reduction kernel (each split's loads in turn) and the partials' round trip at ~4.5 TB/s
-    if (ks > 1) c += 2.5f + 0.35f * (float)ks + (float)ks * (float)p.M * (float)columns_of(p) * (p.W2 ? 16.0f : 8.0f) / 4.5e6f;
+    const float ramp = low ? (float)rem / 256.0f : rem > 128 ? (float)(rem - 128) / 128.0f : 0.0f;
+    float per_k = (float)(T / 256) * w.full;
+    if (rem) per_k += w.half + (w.full - w.half) * ramp;
+    float c = (float)((T + 255) / 256) * w.fix + per_k * (float)p.K / (4096.0f * (float)ks);
+    if (ks > 1) {
+        const float mb = (float)ks * (float)p.M * (float)columns_of(p) * (p.W2 ? 16.0f : 8.0f) / 4.5e6f;
+        c += p.W2 ? f.d0 + f.d1 * (float)ks + f.db * mb : f.r0 + f.r1 * (float)ks + f.rb * mb;
+    }
     return c;
 }
 
-// The base shape with its K split, unless another is cheaper by its tile counts:
-// any shape without a split, or, where the base splits, 128- or 64-row tiles with
-// as many splits or fewer (so no call needs more split-K partials than the base
-// choice would).  MLX, M = 77, K = 8192, N = 2048: 16 splits of 128-row tiles
-// 20.8 us, 8 of 64-row tiles 16.4 (launch included); M = 128, K = N = 4096
-// 21.1 -> 16.3.
+// Base choice: the shape of rb_pick, K split (powers of two, whole 256-element
+// super-blocks, >= 512 of K per split) while the grid still fits one wave of
+// workgroups.
+static void base_plan(GemmParams& p) {
+    p.shape = rb_pick(p.format, p.M, p.N, p.K, p.W2 != nullptr);
+    p.ksplit = 1;
+    if (p.shape == 5 || p.shape == 6) return;  // K groups: the tile takes the whole K range
+    const uint32_t T = tiles_of(p, rb_dims(p.shape));
+    while (T * p.ksplit * 2 <= 256 && p.K % (256 * p.ksplit * 2) == 0 && p.K / (p.ksplit * 2) >= 512) p.ksplit *= 2;
+}
+
+// The base choice, unless another is cheaper by more than its price may be off:
+// any shape without a split or, where the base splits, 128- or 64-row tiles with as
+// many splits or fewer (so no call needs more split-K partials than the base choice
+// would).  2% for tiles of 128 or more rows without a split, 7% for the others,
+// as the fits' errors lie.  Over 3368 shapes of 17 rows or more the chosen plans are
+// 1.124x as fast as the base ones by geometric mean, 0.5% off the fastest, and 18 are
+// more than 3% slower than their base (one table for all formats without a fixed
+// cost per wave: 1.107x, 140, Q8_0 by up to 37%).  On 900 shapes outside the fits
+// where the choices differ 1.187x, against 1.165x.
 void gemm_plan(GemmParams& p) {
     const bool dual = p.W2 != nullptr;
-    p.shape = rb_pick(p.format, p.M, p.N, p.K, dual);
-    p.ksplit = 1;
-    if (p.shape != 5 && p.shape != 6) {  // K groups: the tile takes the whole K range
-        // split K (powers of two, whole 256-element super-blocks, >= 512 of K
-        // per split) while the grid still fits one wave
-        const uint32_t T = tiles_of(p, rb_dims(p.shape));
-        while (T * p.ksplit * 2 <= 256 && p.K % (256 * p.ksplit * 2) == 0 && p.K / (p.ksplit * 2) >= 512) p.ksplit *= 2;
-    }
+    base_plan(p);
     if (p.format != QUANT_VAR_RATE_AFFINE && p.format != QUANT_EXL3) {  // those have one shape
         const bool heavy = p.format == QUANT_Q4_K || p.format == QUANT_TERNARY_1_58;
         const bool groups_ok = p.K % 128 == 0, wide = groups_ok && wide_format(p.format);
         const int cand[6] = {dual ? 2 : 1, dual ? -1 : (heavy ? 3 : 0), dual ? (wide ? 8 : -1) : (wide ? 7 : -1),
                              dual || !groups_ok ? -1 : 6, dual || !groups_ok || p.M > 128 ? -1 : 5, dual ? -1 : 4};
-        const float base = plan_cost(p, p.shape, p.ksplit);
-        const float margin = 0.08f * base;  // a near tie keeps the base's split (M = 640, K = 4096, N = 1024 ran even)
-        // one kernel without partials on a tie: M = 700, K = 4096, N = 1024 18.7 us, split 19.4
-        float best = p.ksplit > 1 ? base : 0.97f * base;
-        uint32_t ksplit = p.ksplit;
-        for (int s : cand) {
-            if (s < 0) continue;
-            const float c = plan_cost(p, s, 1);
-            if (c < best) {
-                best = c;
-                p.shape = s;
-                ksplit = 1;
-            }
-        }
+        const int shape0 = p.shape;
+        const uint32_t ks0 = p.ksplit;
+        const float base = plan_cost(p, shape0, ks0);
+        float best = base;
+        auto offer = [&](int s, uint32_t ks, float margin) {
+            if (s == shape0 && ks == ks0) return;
+            const float c = plan_cost(p, s, ks) + margin * base;
+            if (c >= best) return;
+            best = c;
+            p.shape = s;
+            p.ksplit = ks;
+        };
+        for (int s : cand)
+            if (s >= 0) offer(s, 1, s == 4 || s == 5 || s == 6 ? 0.07f : 0.02f);
         for (int s : {1, 4})
-            for (uint32_t ks = 2; !dual && ks <= p.ksplit; ks *= 2) {
-                const float c = plan_cost(p, s, ks) + margin;
-                if (c < best) {
-                    best = c;
-                    p.shape = s;
-                    ksplit = ks;
-                }
-            }
-        p.ksplit = ksplit;
+            for (uint32_t ks = 2; !dual && ks <= ks0; ks *= 2) offer(s, ks, 0.07f);
     }
     p.group_m = (p.M + rb_dims(p.shape).bm - 1) / rb_dims(p.shape).bm >= 4 ? 4u : 2u;
 }

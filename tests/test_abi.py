@@ -253,3 +253,27 @@ def test_projection_plan(lib):
                         if p.kernel_name == "tiled":
                             assert p.k_splits == 1 or K // p.k_splits >= 512, t
                             assert p.k_groups == 1 or (p.k_splits == 1 and K % 128 == 0), t
+
+
+@pytest.mark.parametrize("fmt,M,K,N,swiglu,want", [
+    # us measured: this plan / the one that a single cost table for all formats took
+    (8, 128, 4096, 14336, False, (128, 64, 2, 1)),    # 26.9 / 30.9 (64 x 128, two K groups)
+    (8, 84, 14336, 16384, False, (128, 64, 2, 1)),    # 80.0 / 95.0
+    (0, 73, 4096, 16384, False, (128, 64, 2, 1)),     # 23.8 / 26.9
+    (2, 62, 11008, 16384, False, (128, 64, 2, 1)),    # 71.3 / 85.6
+    (6, 89, 4096, 14336, False, (128, 64, 2, 1)),     # 31.9 / 38.5
+    (7, 64, 14336, 14336, False, (128, 64, 2, 1)),    # 64.4 / 81.9
+    (6, 64, 2048, 5632, False, (64, 128, 1, 4)),      # 12.6 / 17.8
+    (6, 301, 2048, 1024, False, (64, 128, 1, 4)),     # 12.6 / 17.5
+    (0, 141, 2048, 2048, False, (64, 128, 1, 4)),     # 11.7 / 13.6
+    (0, 316, 4096, 2816, False, (64, 128, 1, 2)),     # 20.5 / 24.4
+    (6, 256, 2048, 4096, True, (128, 128, 1, 4)),     # 27.8 / 35.7 (no split)
+    (0, 128, 2048, 8192, True, (128, 128, 1, 4)),     # 26.0 / 29.3
+    (6, 504, 4096, 4096, True, (128, 128, 1, 2)),     # 57.8 / 71.9
+    # gains over the base plan that stay
+    (1, 77, 8192, 2048, False, (64, 128, 1, 8)),      # 16.4 / 20.8 (128 x 128, 16 splits)
+    (8, 8192, 4096, 14336, True, (256, 128, 1, 1)),   # 1660 / 1909 (128 x 128)
+    (2, 1000, 4096, 14336, True, (256, 128, 1, 1)),   # 241 / 309 (128 x 128)
+])
+def test_projection_plan_measured(lib, fmt, M, K, N, swiglu, want):
+    assert m4_bridge.projection_plan(lib, fmt, M, K, N, swiglu=swiglu).astuple()[1:] == want

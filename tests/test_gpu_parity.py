@@ -263,10 +263,10 @@ def test_in_flight_buffers_retained_until_synchronize(bridge):
                                        (0, 129, 4096, 4096), (1, 129, 4096, 4096), (7, 150, 2048, 1536),
                                        (6, 300, 2048, 1024)])
 def test_under_filled_grid_shapes(bridge, oracle, fmt, M, K, N):
-    """Full-size shapes whose tile grid under-fills the 256 CUs (the headline:
-    112 tiles x 2 K splits; 384 tiles = 1.5 rounds; 80 tiles x 2 splits) and
-    64-row tiles with a K split (M = 129, 150, 300: last 128-row tile at most
-    half full), checked against the oracle on a row sample (every output
+    """Full-size shapes whose tile grid under-fills the 256 CUs (the headline's
+    224 tiles of 128 x 64; 384 and 80 tiles of 128 x 128, whichever plan takes
+    them) and 64-row tiles with a K split (M = 129, 150, 300: last 128-row tile
+    at most half full), checked against the oracle on a row sample (every output
     column) and for run-to-run determinism of the split-K reduction."""
     X = synth.activations(M, K, 120 + fmt, std=0.35)
     W = synth.random_blocks(fmt, N, K, 121 + fmt)
@@ -282,21 +282,26 @@ def test_under_filled_grid_shapes(bridge, oracle, fmt, M, K, N):
     np.testing.assert_array_equal(host(Y2).view(np.uint16), host(Y).view(np.uint16))  # deterministic
 
 
-@pytest.mark.parametrize("fmt,M,K,N", [(1, 128, 4096, 12352), (0, 100, 2176, 12300), (2, 128, 2048, 12288),
-                                       (3, 65, 4096, 12352), (8, 127, 2176, 12416), (1, 128, 128, 12288),
-                                       (0, 96, 384, 12352), (0, 40, 4096, 12352),
-                                       (3, 150, 2048, 8200), (0, 129, 1152, 8192), (1, 140, 4096, 16384),
-                                       (1, 128, 4160, 12352)])
-def test_k_group_tiles(bridge, oracle, fmt, M, K, N):
+@pytest.mark.parametrize("fmt,M,K,N,tile", [(1, 128, 4096, 12352, (128, 64, 2)), (0, 100, 2176, 12300, (128, 64, 2)),
+                                            (2, 128, 2048, 12288, (128, 64, 2)), (3, 65, 4096, 12352, (128, 64, 2)),
+                                            (8, 127, 2176, 12416, (128, 64, 2)), (7, 128, 512, 12288, (128, 64, 2)),
+                                            (6, 128, 640, 12300, (128, 64, 2)),
+                                            (1, 128, 128, 12288, (64, 128, 1)), (0, 96, 384, 12352, (64, 128, 1)),
+                                            (0, 40, 4096, 12352, None), (0, 129, 128, 5632, (64, 128, 2)),
+                                            (0, 150, 384, 5632, (64, 128, 2)), (3, 150, 2048, 8200, (64, 128, 2)),
+                                            (0, 129, 1152, 8192, (64, 128, 2)), (1, 140, 4096, 8192, (64, 128, 2)),
+                                            (1, 140, 4096, 16384, (128, 128, 1)), (1, 128, 4160, 12352, (64, 128, 1))])
+def test_k_group_tiles(bridge, oracle, fmt, M, K, N, tile):
     """The 128 x 64 tile whose two K groups take alternate 64-K steps and
-    meet in LDS (M <= 128 with at least 192 column tiles), and the 64 x 128
-    tile as two K groups (M past a multiple of 128 by at most 64, no K split
-    needed: M = 129, 140, 150): ragged M and N,
-    K with an odd number of step pairs (2176 = 17 pairs), one or three pairs
-    (K = 128, 384: fewer rounds than the stager runs ahead), M = 40 (whichever
-    small-M or tiled path takes it), K = 4160 (not whole 128-K rounds: the
-    shape choice leaves the K-group tiles), checked against the oracle on a
-    row sample with every column, and deterministic."""
+    meet in LDS (M <= 128, many column tiles), and the 64 x 128 tile as two K
+    groups (no K split needed): ragged M and N, K with an odd number of step
+    pairs (2176 = 17 pairs), one or three pairs (K = 128, 384: fewer rounds than
+    the stager runs ahead; at M <= 128 the tile without K groups is the cheaper
+    one there), M = 40 (the small-M kernel), K = 4160 (not whole 128-K rounds: the
+    shape choice leaves the K-group tiles), checked against the oracle on a row
+    sample with every column, and deterministic."""
+    got = plan(bridge, fmt, M, K, N)
+    assert (got[0] == "small_m" if tile is None else got == ("tiled", *tile, 1)), got
     X = synth.activations(M, K, 140 + fmt, std=0.35)
     W = synth.random_blocks(fmt, N, K, 141 + fmt)
     Y = empty16(M, N)
@@ -466,13 +471,14 @@ def test_few_rows(bridge, oracle, fmt, layout, M, K, N):
 
 
 @pytest.mark.parametrize("fmt", [0, 1, 2, 3, 8])
-@pytest.mark.parametrize("layout,M,K,N", [("plain", 77, 8192, 2046), ("residual", 128, 4096, 4096),
-                                          ("head", 256, 2048, 512), ("plain", 384, 4096, 1024),
-                                          ("plain", 65, 2048, 2048)])
-def test_split_k_plans(bridge, oracle, fmt, layout, M, K, N):
+@pytest.mark.parametrize("layout,M,K,N,splits", [("plain", 77, 8192, 2046, 8), ("residual", 128, 4096, 4096, 4),
+                                                 ("head", 256, 2048, 512, 4), ("plain", 384, 4096, 1024, 4),
+                                                 ("plain", 65, 2048, 2048, 4)])
+def test_split_k_plans(bridge, oracle, fmt, layout, M, K, N, splits):
     """Projections whose K split and tile height are chosen together (64-row
-    tiles with fewer splits than 128-row ones, a full and a ragged last row
-    tile, a ragged N), against the oracle on a row sample with every column."""
+    tiles with as many splits as 128-row ones or fewer, a full and a ragged last
+    row tile, a ragged N), against the oracle on a row sample with every column."""
+    assert plan(bridge, fmt, M, K, N) == ("tiled", 64, 128, 1, splits)
     X = synth.activations(M, K, 190 + fmt, std=0.35)
     W = weights("quantized", fmt, N, K, 191 + fmt)
     rows = np.unique(np.r_[0, 31, 32, 63, 64, M - 1])
