@@ -222,26 +222,50 @@ static uint32_t column_tiles(const GemmParams& p, uint32_t cw) {
     return t;
 }
 
-// Where this kernel is the fastest (each launch in a graph, us, other kernel ->
-// this one):
-//  * SwiGLU: always, against the 128-row tiles (MLX, K = 4096, N = 14336:
-//    M = 1 33.2 -> 21.3, M = 16 34.0 -> 33.2);
-//  * a layer's Q, K and V in one launch: always (they were three launches);
-//  * formats without a small-M kernel: always (Q8_0 4096 x 4096, M = 1 11.1 ->
-//    6.9, M = 16 14.1 -> 9.4);
-//  * where the small-M kernel needs its K split: up to 8 rows (MLX K = 14336,
-//    N = 4096: M = 1 16.7 -> 11.3, M = 8 18.4 -> 15.5, M = 16 18.3 -> 21.5:
-//    every lane of a row reads its own X lines), up to 16 with few columns (K =
-//    N = 2048: 8.5 -> 4.9), but not past 1024 column tiles, which are not
-//    resident at once (N = 28672, M = 1: 19.2 -> 21.8);
-//  * where it runs as one kernel: one or two rows (MLX 4096 x 4096: M = 1
+// Where this kernel is the fastest.  Every column tile reads all of X from L2, so
+// what it loses on is X bytes (M K per tile) where the other kernels can split K;
+// 3386 shapes of 1 .. 16 rows over all formats, each launch in a graph, us other
+// kernel -> this one:
+//  * SwiGLU, against the 128-row tiles: MLX K = 4096, N = 14336 M = 1 33.2 -> 21.3,
+//    M = 16 34.0 -> 33.2; of 800 shapes 23 below 1.2x, two below even, but for VAR_RATE
+//    against 16 K splits (K = 8192, N = 512 108 -> 145), EXL3 with short K and many
+//    columns (K = 1024, N = 28672 56 -> 65) and Q4_0 past M K = 160 Ki (M = 16, K =
+//    14336, N = 5632 60.5 -> 67.9);
+//  * formats without a small-M kernel, and a layer's Q, K and V in one launch: where
+//    the tiles split K, up to M K = 128 Ki (ternary M = 16, K = 14336, N = 256 14.4 ->
+//    17.7), Q8_0 104 Ki but at 128 to 256 tiles (M = 8, K = 14336, N = 512 19.0 -> 19.8;
+//    M = 9, K = 14336, N = 4096 25.0 -> 21.0), and from nine
+//    rows past one workgroup per CU Q8_0 48 Ki (M = 16, N = 5632: K = 2048 11.3 -> 9.4, K =
+//    4096 14.7 -> 16.1) and PRISM 64 Ki (N = 8192: M = 16, K = 4096 1.04x, M = 11, K =
+//    8192 18.8 -> 20.7); VAR_RATE and EXL3 always (M = 16, K = 14336, N = 1536 1.6x);
+//  * where the small-M kernel splits K: up to 128 column tiles M K <= 96 Ki (M = 12, K =
+//    14336, N = 2048 MLX 14.1 -> 17.7), Q4_K 128 Ki (M = 8 16.8 -> 15.3); past that eight
+//    rows (MLX K = 14336, N = 4096, M = 8 19.3 -> 17.2); past one workgroup per CU (256
+//    tiles) only what K makes up for the uneven load: MLX and g64 below K = 8192 (g64 M =
+//    2, N = 11008: K = 4096 even, K = 8192 19.5 -> 23.0), Q4_0 to M K = 48 Ki; not past
+//    1024 tiles, which are not resident at once (N = 28672, M = 1: 19.2 -> 21.8);
+//  * where that runs as one kernel: one or two rows (MLX 4096 x 4096: M = 1
 //    5.5 -> 4.8, M = 2 5.6 -> 5.1, M = 4 5.6 -> 5.7), Q4_K up to 8 (8.2 -> 6.2).
 bool gemv_fits(const GemmParams& p) {
     if (p.M > 16 || p.K % 256) return false;
-    if (p.W2 || p.ngroups > 1 || !skinny_supported(p)) return true;
-    const uint32_t tiles = (p.N + 15) / 16;
-    if (skinny_one_kernel(p)) return p.M <= (p.format == QUANT_Q4_K ? 8u : 2u);
-    return tiles <= 1024 && (p.M <= 8 || tiles <= 128);
+    const uint32_t tiles = column_tiles(p, 16);
+    auto mk_upto = [&](uint32_t ki) { return (uint64_t)p.M * p.K <= (uint64_t)ki << 10; };
+    const int f = p.format;
+    if (p.W2 || p.ngroups > 1 || !skinny_supported(p)) {
+        const uint32_t ks = gemm_base_ksplit(p);
+        if (p.W2)
+            return !(f == QUANT_VAR_RATE_AFFINE && ks >= 16) && !(f == QUANT_EXL3 && p.K <= 1024 && tiles > 768) &&
+                   !(f == QUANT_Q4_0 && ks > 1 && tiles > 256 && !mk_upto(160));
+        if (f == QUANT_VAR_RATE_AFFINE || f == QUANT_EXL3) return true;
+        if (ks == 1 && (f != QUANT_Q8_0 || tiles <= 1024)) return true;
+        if (p.M > 8 && tiles > 256 && ks >= 4 && (f == QUANT_Q8_0 || f == QUANT_PRISM_Q2_0)) return mk_upto(f == QUANT_Q8_0 ? 48 : 64);
+        return mk_upto(f == QUANT_Q8_0 && (tiles < 128 || tiles > 256) ? 104 : 128);
+    }
+    if (skinny_one_kernel(p)) return p.M <= (f == QUANT_Q4_K ? 8u : 2u);
+    if (tiles <= 128) return mk_upto(f == QUANT_Q4_K ? 128 : 96);
+    if (tiles > 1024 || p.M > 8) return false;
+    if (tiles <= 256 || f == QUANT_Q4_K || f == QUANT_TERNARY_1_58) return true;
+    return f == QUANT_Q4_0 ? mk_upto(48) : p.K < 8192;
 }
 
 // Two column tiles per workgroup when the workgroups of one would not be

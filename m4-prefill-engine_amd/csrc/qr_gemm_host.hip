@@ -237,6 +237,12 @@ static void base_plan(GemmParams& p) {
     while (T * p.ksplit * 2 <= 256 && p.K % (256 * p.ksplit * 2) == 0 && p.K / (p.ksplit * 2) >= 512) p.ksplit *= 2;
 }
 
+uint32_t gemm_base_ksplit(const GemmParams& p0) {
+    GemmParams p = p0;
+    base_plan(p);
+    return p.ksplit;
+}
+
 // The base choice, unless another is cheaper by more than its price may be off:
 // any shape without a split or, where the base splits, 128- or 64-row tiles with as
 // many splits or fewer (so no call needs more split-K partials than the base choice

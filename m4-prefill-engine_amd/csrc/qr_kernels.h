@@ -34,6 +34,8 @@ struct GemmParams {
 
 // Tile shape, K split and tile order of p (before launch_gemm).
 void gemm_plan(GemmParams& p);
+// K split of gemm_plan's base choice (the most that it would split p).
+uint32_t gemm_base_ksplit(const GemmParams& p);
 hipError_t launch_gemm(const GemmParams& p, hipStream_t st);
 size_t gemm_workspace_floats(const GemmParams& p);
 // Sums split-K partials ws [ks][dual ? 2 : 1][M][N] in split order and writes

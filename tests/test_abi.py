@@ -277,3 +277,30 @@ def test_projection_plan(lib):
 ])
 def test_projection_plan_measured(lib, fmt, M, K, N, swiglu, want):
     assert m4_bridge.projection_plan(lib, fmt, M, K, N, swiglu=swiglu).astuple()[1:] == want
+
+
+@pytest.mark.parametrize("fmt,M,K,N,swiglu,few", [
+    # us measured: the kernel asked for / the other (few rows: one kernel of 16-column strips)
+    (8, 4, 14336, 11008, False, False),   # 29.0 / 40.2
+    (8, 2, 8192, 11008, False, False),    # 19.5 / 23.0
+    (1, 8, 14336, 5632, False, False),    # 22.4 / 31.4
+    (1, 12, 14336, 2048, False, False),   # 14.1 / 17.7
+    (3, 16, 14336, 256, False, False),    # 14.4 / 17.7
+    (6, 16, 14336, 5632, False, False),   # 39.9 / 49.2
+    (7, 11, 8192, 8192, False, False),    # 18.8 / 20.7
+    (4, 8, 8192, 256, True, False),       # 107.7 / 143.0
+    (5, 3, 1024, 28672, True, False),     # 56.3 / 65.2
+    (0, 16, 14336, 5632, True, False),    # 60.5 / 67.9
+    (6, 9, 14336, 4096, False, True),     # 21.0 / 25.0
+    (8, 4, 4096, 14336, False, True),     # 13.0 / 14.2
+    (1, 8, 14336, 4096, False, True),     # 17.2 / 19.3
+    (2, 8, 14336, 2048, False, True),     # 15.3 / 16.8
+    (3, 8, 8192, 16384, False, True),     # 21.7 / 26.2
+    (6, 16, 2048, 5632, False, True),     # 9.4 / 11.3
+    (6, 11, 5632, 6144, False, True),     # 16.7 / 29.7
+    (4, 4, 14336, 14336, True, True),     # 1.7x
+    (1, 1, 4096, 14336, True, True),      # 21.3 / 33.2
+])
+def test_projection_plan_few_rows(lib, fmt, M, K, N, swiglu, few):
+    got = m4_bridge.projection_plan(lib, fmt, M, K, N, swiglu=swiglu).kernel_name
+    assert (got == "few_rows") == few, got
