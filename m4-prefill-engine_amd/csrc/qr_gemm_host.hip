@@ -247,8 +247,9 @@ uint32_t gemm_base_ksplit(const GemmParams& p0) {
 // any shape without a split or, where the base splits, 128- or 64-row tiles with as
 // many splits or fewer (so no call needs more split-K partials than the base choice
 // would).  2% for tiles of 128 or more rows without a split, 7% for the others,
-// as the fits' errors lie.  Over 3368 shapes of 17 rows or more the chosen plans are
-// 1.124x as fast as the base ones by geometric mean, 0.5% off the fastest, and 18 are
+// as the fits' errors lie, 12% for fewer splits of more than 2048 of K each (Q4_0, M =
+// 128, K = 14336, N = 4096: 8 splits of 128 rows 29.9 us, 4 of 64 33.6).  Over 3368 shapes of 17 rows or more the chosen plans are
+// 1.124x as fast as the base ones by geometric mean, 0.5% off the fastest, and 16 are
 // more than 3% slower than their base (one table for all formats without a fixed
 // cost per wave: 1.107x, 140, Q8_0 by up to 37%).  On 900 shapes outside the fits
 // where the choices differ 1.187x, against 1.165x.
@@ -275,7 +276,8 @@ void gemm_plan(GemmParams& p) {
         for (int s : cand)
             if (s >= 0) offer(s, 1, s == 4 || s == 5 || s == 6 ? 0.07f : 0.02f);
         for (int s : {1, 4})
-            for (uint32_t ks = 2; !dual && ks <= ks0; ks *= 2) offer(s, ks, 0.07f);
+            for (uint32_t ks = 2; !dual && ks <= ks0; ks *= 2)
+                offer(s, ks, ks < ks0 && p.K / ks > 2048 ? 0.12f : 0.07f);
     }
     p.group_m = (p.M + rb_dims(p.shape).bm - 1) / rb_dims(p.shape).bm >= 4 ? 4u : 2u;
 }

@@ -267,6 +267,7 @@ def test_projection_plan(lib):
     (6, 301, 2048, 1024, False, (64, 128, 1, 4)),     # 12.6 / 17.5
     (0, 141, 2048, 2048, False, (64, 128, 1, 4)),     # 11.7 / 13.6
     (0, 316, 4096, 2816, False, (64, 128, 1, 2)),     # 20.5 / 24.4
+    (0, 128, 14336, 4096, False, (128, 128, 1, 8)),   # 29.9 (4 splits of 64-row tiles: 33.6)
     (6, 256, 2048, 4096, True, (128, 128, 1, 4)),     # 27.8 / 35.7 (no split)
     (0, 128, 2048, 8192, True, (128, 128, 1, 4)),     # 26.0 / 29.3
     (6, 504, 4096, 4096, True, (128, 128, 1, 2)),     # 57.8 / 71.9
