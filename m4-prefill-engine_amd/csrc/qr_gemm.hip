@@ -698,8 +698,10 @@ static hipError_t rb_launch_fmt(const GemmParams& p, hipStream_t st) {
         return rb_launch_cfg<F, QR_RB_MID, false>(p, st);  // the only shape for these formats
     } else {
         switch (p.shape) {
-            case 0: return rb_launch_cfg<F, QR_RB_BIG, false>(p, st);
-            case 3: return rb_launch_cfg<F, QR_RB_BIG_K, false>(p, st);
+            case 0:
+            case 3:  // 3 for the formats that pay for two waves per SIMD, 0 for the others
+                if constexpr (big_k_format(F)) return rb_launch_cfg<F, QR_RB_BIG_K, false>(p, st);
+                else return rb_launch_cfg<F, QR_RB_BIG, false>(p, st);
             case 4: return rb_launch_cfg<F, QR_RB_MID64, false>(p, st);
             case 5: return rb_launch_cfg<F, QR_RB_KG, false>(p, st);
             case 6: return rb_launch_cfg<F, QR_RB_MID64_KG, false>(p, st);

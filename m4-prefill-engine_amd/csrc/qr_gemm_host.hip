@@ -257,9 +257,8 @@ void gemm_plan(GemmParams& p) {
     const bool dual = p.W2 != nullptr;
     base_plan(p);
     if (p.format != QUANT_VAR_RATE_AFFINE && p.format != QUANT_EXL3) {  // those have one shape
-        const bool heavy = p.format == QUANT_Q4_K || p.format == QUANT_TERNARY_1_58;
         const bool groups_ok = p.K % 128 == 0, wide = groups_ok && wide_format(p.format);
-        const int cand[6] = {dual ? 2 : 1, dual ? -1 : (heavy ? 3 : 0), dual ? (wide ? 8 : -1) : (wide ? 7 : -1),
+        const int cand[6] = {dual ? 2 : 1, dual ? -1 : (big_k_format(p.format) ? 3 : 0), dual ? (wide ? 8 : -1) : (wide ? 7 : -1),
                              dual || !groups_ok ? -1 : 6, dual || !groups_ok || p.M > 128 ? -1 : 5, dual ? -1 : 4};
         const int shape0 = p.shape;
         const uint32_t ks0 = p.ksplit;

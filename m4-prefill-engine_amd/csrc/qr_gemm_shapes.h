@@ -40,6 +40,8 @@ struct RbShape {
 constexpr bool wide_format(int f) {
     return f == QUANT_Q4_0 || f == QUANT_MLX_4BIT || f == QUANT_Q4_K || f == QUANT_TERNARY_1_58 || f == QUANT_MLX_4BIT_G64;
 }
+// Formats whose 128 x 256 tiles are shape 3 (8 waves), not 0.
+constexpr bool big_k_format(int f) { return f == QUANT_Q4_K || f == QUANT_TERNARY_1_58; }
 // Base shape choice (gemm_plan compares it with the others by tile count).  At M >= 1024 the wide tile is used while it alone fills the
 // 256 CUs; when it cannot (N small), 128 x 128 tiles give twice the tiles, so
 // the K split -- whose fp32 partials are M x N x 4 bytes written and read per
@@ -56,7 +58,7 @@ inline int rb_pick(int format, uint32_t M, uint32_t N, uint32_t K, bool dual) {
         // the heavier decodes (Q4_K's fp32 affine, ternary's 2-bit fields) run
         // best as two waves per SIMD, one decoding while the other multiplies
         // (ternary M = 2048: 68-70 us vs 76 us with one wave per SIMD)
-        if (format == QUANT_Q4_K || format == QUANT_TERNARY_1_58) return 3;
+        if (big_k_format(format)) return 3;
         const uint32_t big_tiles = ((M + 127) / 128) * ((N + 255) / 256);
         if (big_tiles < 256) return 1;
         return 0;

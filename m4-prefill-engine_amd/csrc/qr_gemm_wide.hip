@@ -175,8 +175,7 @@ __global__ void __launch_bounds__(wide::kThreads, 1) gemm_wide_kernel(GemmParams
     uint32_t tmi, tni;
     tile_of(bid, nt_m, nt_n, p.group_m, tmi, tni);
     const int m0 = tmi * BM, n0 = tni * BNO;
-    const uint32_t ksplit = p.ksplit ? p.ksplit : 1, kz = blockIdx.y;
-    const uint32_t nsteps = K / ksplit / 32, g_begin = kz * nsteps;
+    const uint32_t nsteps = K / 32;
     const uint32_t col_bytes = (uint32_t)p.col_bytes;
     const int mrows = min(BM, (int)M - m0), ncols = min(BNO, (int)N - n0);
 
@@ -195,7 +194,7 @@ __global__ void __launch_bounds__(wide::kThreads, 1) gemm_wide_kernel(GemmParams
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)smem);
     const uint32_t xdst = lds0 + (uint32_t)(XCP * wave) * 1024u;
     auto issue_x = [&](uint32_t pair, int f, uint32_t xoff, int q) {
-        const uint32_t soff = (g_begin + 2u * min(pair, nsteps / 2 - 1)) * 64u;
+        const uint32_t soff = 2u * min(pair, nsteps / 2 - 1) * 64u;
         wide::copy_lds(xdst + xoff + (uint32_t)(f * (XSLOT / 2) + q * 1024), xo[f][q], xr, soff);
     };
 
@@ -204,7 +203,7 @@ __global__ void __launch_bounds__(wide::kThreads, 1) gemm_wide_kernel(GemmParams
     // DUAL: columns 128 w .. + 63 are gate columns 64 w .. + 63, the next 64 the up columns.
     uint8_t* const wring = smem + XR * XSLOT;
     uint8_t* const wraw = wring + WR * WSLOT;
-    const uint32_t nrounds = nsteps / wide::kRG, r_begin = g_begin / wide::kRG;
+    const uint32_t nrounds = nsteps / wide::kRG;
     const u4_t wrs = wide::scalar_rsrc((DUAL && (wave & 1) ? p.W2 : p.W) + (size_t)n0 * col_bytes, (uint32_t)ncols * col_bytes);
     // copy q of this wave: units 64 (NU wave + q) + lane, i.e. columns 64 wave .. + 63
     uint32_t wo[NU], wodd[F == QUANT_Q4_K ? NU : 1];
@@ -217,7 +216,7 @@ __global__ void __launch_bounds__(wide::kThreads, 1) gemm_wide_kernel(GemmParams
     }
     const uint32_t wrawdst = lds0 + (uint32_t)(XR * XSLOT + WR * WSLOT + NU * wave * 1024);
     auto issue_w = [&](uint32_t rd, int q) {
-        const uint32_t r = r_begin + min(rd, nrounds - 1);
+        const uint32_t r = min(rd, nrounds - 1);
         const uint32_t soff = F == QUANT_Q4_K ? (r >> 1) * 144u : r * (uint32_t)RD::kBytes;
         uint32_t vo = wo[q];
         if constexpr (F == QUANT_Q4_K) vo += (r & 1u) ? wodd[q] : 0u;
@@ -238,7 +237,7 @@ __global__ void __launch_bounds__(wide::kThreads, 1) gemm_wide_kernel(GemmParams
     // half is named and the rest dropped by the compiler.
     auto decode_w = [&](uint32_t rd, int g, int q, uint32_t o[16]) {
         uint32_t raw[Dec::kRawWords], t[8];
-        const uint32_t par = RD::group(rw, g, r_begin + rd, raw);
+        const uint32_t par = RD::group(rw, g, rd, raw);
         decode_half_fast<F>(raw, par, q >> 2, t);
         o[2 * q] = t[2 * (q & 3)];
         o[2 * q + 1] = t[2 * (q & 3) + 1];
@@ -252,7 +251,7 @@ __global__ void __launch_bounds__(wide::kThreads, 1) gemm_wide_kernel(GemmParams
     auto fix_w = [&](uint32_t rd, int g, int woff) {
         if constexpr (F == QUANT_Q4_K || F == QUANT_Q4_0) {
             uint32_t raw[Dec::kRawWords];
-            const uint32_t par = RD::group(rw, g, r_begin + rd, raw);
+            const uint32_t par = RD::group(rw, g, rd, raw);
             const bool slow = needs_exact<F>(raw, par);
             if (__any(slow)) {
                 uint32_t ex[16];
@@ -410,8 +409,7 @@ __global__ void __launch_bounds__(wide::kThreads, 1) gemm_wide_kernel(GemmParams
     // ---- epilogue, one 32-row band of the wave tile at a time through LDS:
     // accumulator element r of lane l is row 8 (r / 4) + 4 (l / 32) + r % 4,
     // column l % 32 of its 32 x 32 tile; a lane then owns 8 consecutive columns
-    // of one row.  K split: fp32 partials [split][plane][M][N] (plane 1: the
-    // SwiGLU up projection), summed by splitk_reduce_kernel. ----
+    // of one row. ----
     const int r0 = m0 + 32 * TM * wr, c0 = n0 + 32 * NJ * wc;
     const bool vec_io = ((reinterpret_cast<uintptr_t>(p.Y) | reinterpret_cast<uintptr_t>(p.R)) & 15u) == 0 &&
                         (N & 7u) == 0 && (p.head_D & 7u) == 0;
@@ -456,25 +454,6 @@ __global__ void __launch_bounds__(wide::kThreads, 1) gemm_wide_kernel(GemmParams
                 for (int q = 0; q < 8; q++) u[q] = uu[q];
             }
             const int cnt = min(8, (int)N - n);
-            if (ksplit > 1) {
-                const size_t plane = (size_t)M * N;
-                float* o = p.ws + (size_t)kz * plane * (DUAL ? 2 : 1) + (size_t)m * N + n;
-                if ((N & 3u) == 0) {  // cnt is 4 or 8 and o is 16-byte aligned
-                    for (int q = 0; q < cnt; q += 4) {
-                        *reinterpret_cast<f4_t*>(o + q) = q ? f4_t{v[4], v[5], v[6], v[7]} : f4_t{v[0], v[1], v[2], v[3]};
-                        if constexpr (DUAL)
-                            *reinterpret_cast<f4_t*>(o + plane + q) = q ? f4_t{u[4], u[5], u[6], u[7]} : f4_t{u[0], u[1], u[2], u[3]};
-                    }
-                } else {
-#pragma unroll
-                    for (int q = 0; q < 8; q++) {
-                        if (q >= cnt) continue;
-                        o[q] = v[q];
-                        if constexpr (DUAL) o[plane + q] = u[q];
-                    }
-                }
-                continue;
-            }
             if constexpr (DUAL) {
 #pragma unroll
                 for (int q = 0; q < 8; q++) v[q] = silu_mul(v[q], u[q]);
@@ -515,13 +494,12 @@ static hipError_t wide_launch(const GemmParams& p, hipStream_t st) {
     const uint32_t ntm = (p.M + C::BM - 1) / C::BM;
     uint32_t T = ntm * ((p.N + BNO - 1) / BNO);
     for (uint32_t g = 1; g < p.ngroups && g < 3; g++) T += ntm * ((p.Nx[g - 1] + BNO - 1) / BNO);
-    const uint32_t ks = p.ksplit ? p.ksplit : 1;
     constexpr int lds = C::template lds_bytes<wide::Round<F>::kUnits>();
-    if (p.K % (128 * ks)) return hipErrorInvalidValue;
+    if (p.K % 128 || p.ksplit > 1) return hipErrorInvalidValue;  // gemm_plan never asks for these
     static size_t attr[kMaxDevices] = {};
     const hipError_t e = lds_limit_once((const void*)kern, lds, attr);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3(T, ks), dim3(wide::kThreads), lds, st, p);
+    hipLaunchKernelGGL(kern, dim3(T), dim3(wide::kThreads), lds, st, p);
     return hipGetLastError();
 }
 
