@@ -281,19 +281,6 @@ constexpr int kLmBytes = 2048;  // row sums and maxima of the merge
 // -infinity would make the whole row NaN).
 constexpr float kNoScore = -3.402823466e38f;
 
-// 1 KB global -> LDS copy (16 bytes per lane, lane l to lds_addr + 16 l); not
-// known to the compiler, so every reader waits for it explicitly.
-__device__ __forceinline__ void attn_copy(uint32_t lds_addr, uint32_t voff, u4_t rsrc, uint32_t soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :: "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(rsrc),
-                    "s"(__builtin_amdgcn_readfirstlane(soff)) : "m0");
-}
-__device__ __forceinline__ u4_t attn_rsrc(const void* base, uint32_t bytes) {
-    const uint64_t a = reinterpret_cast<uint64_t>(base);
-    return u4_t{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a),
-                (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu),
-                (uint32_t)__builtin_amdgcn_readfirstlane(bytes), (uint32_t)kBufferFlags};
-}
 __device__ __forceinline__ float max3(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
 
 template <int D, int NK>  // NK: key groups; 4 / NK blocks of 32 queries per workgroup
@@ -327,8 +314,8 @@ __global__ void __launch_bounds__(256, 2) flash_attn_kernel(AttnParams p, int pa
     const size_t head_elems = (size_t)M * D;
     const int hk = p.Hkv ? h / ((int)p.H / (int)p.Hkv) : h;
     const uint32_t cbytes = (uint32_t)((size_t)Mp * D * 2);
-    const u4_t kr = attn_rsrc(p.Kf + (size_t)hk * Mp * D, cbytes);
-    const u4_t vr = attn_rsrc(p.Vtf + (size_t)hk * Mp * D, cbytes);
+    const u4_t kr = scalar_rsrc(p.Kf + (size_t)hk * Mp * D, cbytes);
+    const u4_t vr = scalar_rsrc(p.Vtf + (size_t)hk * Mp * D, cbytes);
     const auto qr_ = make_rsrc(p.Q + (size_t)h * head_elems, (uint32_t)(head_elems * 2));
 
     // ---- tile copies.  K rows (keys) hold KU 16-byte units, V^T rows (dims) VU;
@@ -355,8 +342,8 @@ __global__ void __launch_bounds__(256, 2) flash_attn_kernel(AttnParams p, int pa
         const bool part = k0 + KT > (uint32_t)Mp;  // a V^T chunk past Mp would be the next dim's first keys
 #pragma unroll
         for (int q = 0; q < CPW; q++) {
-            attn_copy(dst + q * 1024u, ko[q] + k0 * D * 2u, kr, 0);  // rows past Mp: past the head's cache
-            attn_copy(dst + KB + q * 1024u, part && k0 + vk[q] >= (uint32_t)Mp ? kOOB : vo[q], vr, k0 * 2u);
+            copy_lds(dst + q * 1024u, ko[q] + k0 * D * 2u, kr, 0);  // rows past Mp: past the head's cache
+            copy_lds(dst + KB + q * 1024u, part && k0 + vk[q] >= (uint32_t)Mp ? kOOB : vo[q], vr, k0 * 2u);
         }
     };
 

@@ -27,6 +27,20 @@ constexpr uint32_t kOOB = 0x80000000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, kBufferFlags);
 }
+// The same descriptor from a wave-uniform base, as scalar words for inline asm.
+__device__ __forceinline__ u4_t scalar_rsrc(const void* base, uint32_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    return u4_t{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a),
+                (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu),
+                (uint32_t)__builtin_amdgcn_readfirstlane(bytes), (uint32_t)kBufferFlags};
+}
+// 1 KB global -> LDS copy (16 bytes per lane, lane l to lds_addr + 16 l).  The
+// compiler does not know of it, so every reader waits for it explicitly.
+__device__ __forceinline__ void copy_lds(uint32_t lds_addr, uint32_t voff, u4_t rsrc, uint32_t soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :: "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(rsrc),
+                    "s"(__builtin_amdgcn_readfirstlane(soff)) : "m0");
+}
 __device__ __forceinline__ uint32_t ld_b32(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
 }

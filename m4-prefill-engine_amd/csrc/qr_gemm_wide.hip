@@ -57,27 +57,12 @@ __device__ __forceinline__ uint32_t swz(uint32_t r) { return ((r >> 2) & 3u) ^ (
 // 128-byte rows (X of a pair of steps): unit u of row r at u ^ xswz(r).
 __device__ __forceinline__ uint32_t xswz(uint32_t r) { return (r ^ (r >> 3)) & 7u; }
 
-// Buffer descriptor of `bytes` from a wave-uniform base, as scalar words.
-__device__ __forceinline__ u4_t scalar_rsrc(const void* base, uint32_t bytes) {
-    const uint64_t a = reinterpret_cast<uint64_t>(base);
-    return u4_t{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a),
-                (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32) & 0xffffu),
-                (uint32_t)__builtin_amdgcn_readfirstlane(bytes), (uint32_t)kBufferFlags};
-}
-
-// 1 KB global -> LDS copy (16 bytes per lane).
-__device__ __forceinline__ void copy_lds(uint32_t lds_addr, uint32_t voff, u4_t rsrc, uint32_t soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :: "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(rsrc),
-                    "s"(__builtin_amdgcn_readfirstlane(soff)) : "m0");
-}
-
 // The packed bytes of one column for one round of 4 steps (128 K), as kUnits
 // 16-byte units copied to LDS.  off(u) is unit u's byte offset from the round's
-// start in the column; word() maps word w of the round's bytes to its place in
-// the units (72-byte rounds: the last unit is bytes 56..71, so that nothing
-// past the round is read); group() picks the raw words that decode_half_fast
-// takes for group g of the round, and returns its parity argument.
+// start in the column (72-byte rounds: the last unit is bytes 56..71, so that
+// nothing past the round is read, and words 16.. of the units are two on from the
+// round's); group() picks the raw words that decode_half_fast takes for group g of
+// the round, and returns its parity argument.
 constexpr int kRG = 4;
 template <int F> struct Round;
 template <> struct Round<QUANT_Q4_0> {
@@ -182,7 +167,7 @@ __global__ void __launch_bounds__(wide::kThreads, 1) gemm_wide_kernel(GemmParams
     // ---- X copies: a pair of steps is 128 bytes of every row (whole cache
     // lines), copied in two halves of the rows; copy q of this wave fills rows
     // 8 (XCP wave + q) .. + 7 of its half ----
-    const u4_t xr = wide::scalar_rsrc(p.X + (size_t)m0 * K, (uint32_t)mrows * K * 2u);
+    const u4_t xr = scalar_rsrc(p.X + (size_t)m0 * K, (uint32_t)mrows * K * 2u);
     uint32_t xo[2][XCP];
 #pragma unroll
     for (int f = 0; f < 2; f++)
@@ -195,7 +180,7 @@ __global__ void __launch_bounds__(wide::kThreads, 1) gemm_wide_kernel(GemmParams
     const uint32_t xdst = lds0 + (uint32_t)(XCP * wave) * 1024u;
     auto issue_x = [&](uint32_t pair, int f, uint32_t xoff, int q) {
         const uint32_t soff = 2u * min(pair, nsteps / 2 - 1) * 64u;
-        wide::copy_lds(xdst + xoff + (uint32_t)(f * (XSLOT / 2) + q * 1024), xo[f][q], xr, soff);
+        copy_lds(xdst + xoff + (uint32_t)(f * (XSLOT / 2) + q * 1024), xo[f][q], xr, soff);
     };
 
     // ---- weights: a round's packed bytes are copied to LDS (column after
@@ -204,7 +189,7 @@ __global__ void __launch_bounds__(wide::kThreads, 1) gemm_wide_kernel(GemmParams
     uint8_t* const wring = smem + XR * XSLOT;
     uint8_t* const wraw = wring + WR * WSLOT;
     const uint32_t nrounds = nsteps / wide::kRG;
-    const u4_t wrs = wide::scalar_rsrc((DUAL && (wave & 1) ? p.W2 : p.W) + (size_t)n0 * col_bytes, (uint32_t)ncols * col_bytes);
+    const u4_t wrs = scalar_rsrc((DUAL && (wave & 1) ? p.W2 : p.W) + (size_t)n0 * col_bytes, (uint32_t)ncols * col_bytes);
     // copy q of this wave: units 64 (NU wave + q) + lane, i.e. columns 64 wave .. + 63
     uint32_t wo[NU], wodd[F == QUANT_Q4_K ? NU : 1];
 #pragma unroll
@@ -220,7 +205,7 @@ __global__ void __launch_bounds__(wide::kThreads, 1) gemm_wide_kernel(GemmParams
         const uint32_t soff = F == QUANT_Q4_K ? (r >> 1) * 144u : r * (uint32_t)RD::kBytes;
         uint32_t vo = wo[q];
         if constexpr (F == QUANT_Q4_K) vo += (r & 1u) ? wodd[q] : 0u;
-        wide::copy_lds(wrawdst + (uint32_t)q * 1024u, vo, wrs, soff);
+        copy_lds(wrawdst + (uint32_t)q * 1024u, vo, wrs, soff);
     };
     uint32_t rw[NW];
     auto read_raw = [&]() {
