@@ -584,6 +584,9 @@ def main():
         per["rope"] = bench_rope(b, timer, 32, 2048, 64, 55)
 
     head = per.get("cfg2_mlx_m128") or next(iter(per.values()))
+    plan = m4_bridge.projection_plan(b.lib, 1, 128, 4096, 14336)
+    head_kernel = (f"{plan.kernel_name} MLX_4BIT, {plan.tile_rows}x{plan.tile_cols} tiles, {plan.k_groups} K group(s) per "
+                   f"workgroup, {plan.k_splits} K split(s)")
     traffic, traffic_note = (traffic_from_profile("cfg2_mlx_m128") if "cfg2_mlx_m128" in per
                              else (None, "headline not run"))
     out = {
@@ -604,7 +607,7 @@ def main():
         "roofline": {"bound": "mfma", "achieved": head["tflops"], "peak": PEAK_MFMA_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(head["tflops"] / PEAK_MFMA_TFLOPS, 4), "traffic": traffic,
                      "traffic_note": traffic_note,
-                     "kernel": "gemm_rb_kernel<MLX_4BIT, 4, 1, 4, 1, 2> (128x64 tiles, two K groups and a stager wave; one kernel)", "hbm_frac": head.get("frac_hbm")},
+                     "kernel": head_kernel, "hbm_frac": head.get("frac_hbm")},
         "per_config": per,
     }
     if not a.no_probes:

@@ -361,8 +361,9 @@ int gemm_common(void* X, size_t Xb, void* W, size_t Wb, void* Y, size_t Yb, void
 // ---- scratch of the no-allocation projection entry point ----
 // Split-K partials of m4_bridge_dispatch_gemm_noalloc live in this
 // file-scope device array (32 MiB, held on every GPU the library runs on
-// until the process ends): enough for every tiled launch (at most 256
-// workgroups of at most 128 x 256 outputs, so ksplit * M * N <= 8 Mi).  In host code `scratch` names a host-side stand-in
+// until the process ends): enough for every tiled launch (a plan takes no more
+// splits than its base choice, whose split grid is at most 256 workgroups of at
+// most 128 x 256 outputs, so ksplit * M * N <= 8 Mi).  In host code `scratch` names a host-side stand-in
 // only: its device address, per device, comes from hipGetSymbolAddress at
 // init and is the only handle host code passes on.  Nothing in it has to
 // start at zero: every split writes all of its partials before the

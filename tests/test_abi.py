@@ -252,6 +252,8 @@ def test_projection_plan(lib):
                             assert p.k_splits == 1 and p.tile_rows == 256 and K % 128 == 0 and fmt in (0, 1, 2, 3, 8), t
                         if p.kernel_name == "tiled":
                             assert p.k_splits == 1 or K // p.k_splits >= 512, t
+                            # the no-allocation entry point's scratch holds the partials of any plan
+                            assert p.k_splits == 1 or p.k_splits * M * sum(ns) <= 8 << 20, t
                             assert p.k_groups == 1 or (p.k_splits == 1 and K % 128 == 0), t
 
 
