@@ -222,55 +222,98 @@ static uint32_t column_tiles(const GemmParams& p, uint32_t cw) {
     return t;
 }
 
+// Two column tiles per workgroup when the workgroups of one would not be
+// resident at once (MLX N = 14336, K = 4096, M = 1: 15.5 -> 12.8 us).
+uint32_t gemv_tile_columns(const GemmParams& p) { return !p.W2 && column_tiles(p, 16) > 512 ? 32 : 16; }
+
+// ---- the price of this kernel and of the one that would run instead ----
+// us: five terms each, fitted (least squares of the relative error) to ~2300 shapes
+// per format of 1 .. 16 rows, K 1024 .. 14336, N 256 .. 20000, weights read from
+// HBM, launches in a graph; 5 - 7% rms, the tiles' 9 - 12%.
+//  few16, few32 (one and two column tiles per workgroup, each over the widths that
+//      take it): launch, MB of weights, chunks of the longest wave times workgroups
+//      per CU, M K / 1e5 times workgroups per CU (X, which every one of them reads
+//      from L2), M K / 1e5;
+//  split (the small-M kernel with its K split): launch, MB of weights, K per split / 256
+//      times workgroups per CU, partials in 1e6, splits;
+//  tiles (the 128-row tiles): launch, MB of weights, K per split / 256 times
+//      workgroups per CU, the reduction, partials in 1e6.
+struct FewCost {
+    float few16[5], few32[5], split[5], tiles[5];
+};
+static const FewCost& few_cost(int f) {
+    static const FewCost q4_0 = {{2.62f, 0.185f, 0.874f, 4.61f, 1.38f}, {3.31f, 0.238f, 0.794f, 6.52f, 3.38f},
+                                 {6.04f, 0.173f, 0.417f, 2.74f, 0.298f}, {5.39f, 0.163f, 0.88f, 4.28f, 3.28f}};
+    static const FewCost mlx = {{2.6f, 0.164f, 0.944f, 3.49f, 1.54f}, {3.27f, 0.232f, 1.01f, 2.74f, 5.33f},
+                                 {5.89f, 0.168f, 0.365f, 2.45f, 0.283f}, {5.4f, 0.123f, 0.861f, 4.32f, 6.09f}};
+    static const FewCost q4_k = {{3.03f, 0.154f, 0.928f, 2.85f, 1.67f}, {5.73f, 0.2f, 1.35f, 3.61f, 0},
+                                 {6.01f, 0.126f, 0.783f, 2.49f, 0.294f}, {3.63f, 0.175f, 1.38f, 6.49f, 2.77f}};
+    static const FewCost ternary = {{2.82f, 0.192f, 0.775f, 2.71f, 0.974f}, {3.68f, 0.237f, 0.736f, 2.56f, 2.06f},
+                                 {5.99f, 0.229f, 0.325f, 2.46f, 0.304f}, {4.31f, 0.149f, 0.87f, 3.94f, 5.04f}};
+    static const FewCost q8_0 = {{2.62f, 0.136f, 1.34f, 2.03f, 2.63f}, {2.84f, 0.231f, 1.38f, 1.72f, 7.43f},
+                                 {}, {4.07f, 0.173f, 1.08f, 5.55f, 4.11f}};
+    static const FewCost prism = {{2.81f, 0.219f, 0.939f, 2.73f, 0.836f}, {3.32f, 0.36f, 0.874f, 2.6f, 2.04f},
+                                 {}, {4.02f, 0.194f, 0.967f, 4.4f, 3.29f}};
+    static const FewCost g64 = {{2.57f, 0.171f, 0.948f, 3.49f, 1.46f}, {3.24f, 0.242f, 1.02f, 3.03f, 4.02f},
+                                 {5.76f, 0.155f, 0.38f, 2.68f, 0.297f}, {6.09f, 0.166f, 0.858f, 3.79f, 3.14f}};
+    switch (f) {
+        case QUANT_MLX_4BIT: return mlx;
+        case QUANT_Q4_K: return q4_k;
+        case QUANT_TERNARY_1_58: return ternary;
+        case QUANT_Q8_0: return q8_0;
+        case QUANT_PRISM_Q2_0: return prism;
+        case QUANT_MLX_4BIT_G64: return g64;
+        default: return q4_0;
+    }
+}
+static float price(const float* w, float a, float b, float c, float d) { return w[0] + w[1] * a + w[2] * b + w[3] * c + w[4] * d; }
+
 // Where this kernel is the fastest.  Every column tile reads all of X from L2, so
-// what it loses on is X bytes (M K per tile) where the other kernels can split K;
-// 3386 shapes of 1 .. 16 rows over all formats, each launch in a graph, us other
-// kernel -> this one:
+// what it loses on is X bytes where the other kernel can split K, and workgroups that
+// share a CU unevenly; how well the other one splits depends on K (10752 = 42
+// super-blocks splits in two, 8192 in sixteen).  So both are priced, and this one runs where its price
+// is lower by 6%, about the fits' error (this kernel / the other, us): MLX M = 7, K = 7168, N = 8720
+// 24.5 / 18.0, MLX M = 8, K = 14336, N = 5632 31.4 / 22.4, but Q4_K M = 16, K =
+// 10752, N = 1416 14.2 / 45.4, ternary M = 12, K = 13824, N = 3712 15.8 / 37.9.
+// Of 15974 shapes 1.92x the other kernels by geometric mean, 39 more than 3% slower
+// than them (bounds on M K and tiles in its place: 1.84x, 128).
+//  * K up to 1024, below the prices' range: up to 1024 column tiles where the small-M
+//    kernel would run (of 6365 shapes 1.62x, 57 more than 3% slower);
 //  * SwiGLU, against the 128-row tiles: MLX K = 4096, N = 14336 M = 1 33.2 -> 21.3,
 //    M = 16 34.0 -> 33.2; of 800 shapes 23 below 1.2x, two below even, but for VAR_RATE
 //    against 16 K splits (K = 8192, N = 512 108 -> 145), EXL3 with short K and many
 //    columns (K = 1024, N = 28672 56 -> 65) and Q4_0 past M K = 160 Ki (M = 16, K =
 //    14336, N = 5632 60.5 -> 67.9);
-//  * formats without a small-M kernel, and a layer's Q, K and V in one launch: where
-//    the tiles split K, up to M K = 128 Ki (ternary M = 16, K = 14336, N = 256 14.4 ->
-//    17.7), Q8_0 104 Ki but at 128 to 256 tiles (M = 8, K = 14336, N = 512 19.0 -> 19.8;
-//    M = 9, K = 14336, N = 4096 25.0 -> 21.0), and from nine
-//    rows past one workgroup per CU Q8_0 48 Ki (M = 16, N = 5632: K = 2048 11.3 -> 9.4, K =
-//    4096 14.7 -> 16.1) and PRISM 64 Ki (N = 8192: M = 16, K = 4096 1.04x, M = 11, K =
-//    8192 18.8 -> 20.7); VAR_RATE and EXL3 always (M = 16, K = 14336, N = 1536 1.6x);
-//  * where the small-M kernel splits K: up to 128 column tiles M K <= 96 Ki (M = 12, K =
-//    14336, N = 2048 MLX 14.1 -> 17.7), Q4_K 128 Ki (M = 8 16.8 -> 15.3); past that eight
-//    rows (MLX K = 14336, N = 4096, M = 8 19.3 -> 17.2); past one workgroup per CU (256
-//    tiles) only what K makes up for the uneven load: MLX and g64 below K = 8192 (g64 M =
-//    2, N = 11008: K = 4096 even, K = 8192 19.5 -> 23.0), Q4_0 to M K = 48 Ki; not past
-//    1024 tiles, which are not resident at once (N = 28672, M = 1: 19.2 -> 21.8);
-//  * where that runs as one kernel: one or two rows (MLX 4096 x 4096: M = 1
+//  * VAR_RATE and EXL3 projections: always (M = 16, K = 14336, N = 1536 1.6x);
+//  * where the small-M kernel runs as one kernel: one or two rows (MLX 4096 x 4096: M = 1
 //    5.5 -> 4.8, M = 2 5.6 -> 5.1, M = 4 5.6 -> 5.7), Q4_K up to 8 (8.2 -> 6.2).
 bool gemv_fits(const GemmParams& p) {
     if (p.M > 16 || p.K % 256) return false;
-    const uint32_t tiles = column_tiles(p, 16);
-    auto mk_upto = [&](uint32_t ki) { return (uint64_t)p.M * p.K <= (uint64_t)ki << 10; };
     const int f = p.format;
-    if (p.W2 || p.ngroups > 1 || !skinny_supported(p)) {
+    const uint32_t tiles = column_tiles(p, 16);
+    if (p.W2) {
         const uint32_t ks = gemm_base_ksplit(p);
-        if (p.W2)
-            return !(f == QUANT_VAR_RATE_AFFINE && ks >= 16) && !(f == QUANT_EXL3 && p.K <= 1024 && tiles > 768) &&
-                   !(f == QUANT_Q4_0 && ks > 1 && tiles > 256 && !mk_upto(160));
-        if (f == QUANT_VAR_RATE_AFFINE || f == QUANT_EXL3) return true;
-        if (ks == 1 && (f != QUANT_Q8_0 || tiles <= 1024)) return true;
-        if (p.M > 8 && tiles > 256 && ks >= 4 && (f == QUANT_Q8_0 || f == QUANT_PRISM_Q2_0)) return mk_upto(f == QUANT_Q8_0 ? 48 : 64);
-        return mk_upto(f == QUANT_Q8_0 && (tiles < 128 || tiles > 256) ? 104 : 128);
+        return !(f == QUANT_VAR_RATE_AFFINE && ks >= 16) && !(f == QUANT_EXL3 && p.K <= 1024 && tiles > 768) &&
+               !(f == QUANT_Q4_0 && ks > 1 && tiles > 256 && (uint64_t)p.M * p.K > 160u << 10);
     }
-    if (skinny_one_kernel(p)) return p.M <= (f == QUANT_Q4_K ? 8u : 2u);
-    if (tiles <= 128) return mk_upto(f == QUANT_Q4_K ? 128 : 96);
-    if (tiles > 1024 || p.M > 8) return false;
-    if (tiles <= 256 || f == QUANT_Q4_K || f == QUANT_TERNARY_1_58) return true;
-    return f == QUANT_Q4_0 ? mk_upto(48) : p.K < 8192;
+    if (f == QUANT_VAR_RATE_AFFINE || f == QUANT_EXL3) return true;
+    const bool split = p.ngroups <= 1 && skinny_supported(p);
+    if (split && skinny_one_kernel(p)) return p.M <= (f == QUANT_Q4_K ? 8u : 2u);
+    if (p.K <= 1024) return !split || tiles <= (f == QUANT_Q4_K && p.K < 512 ? 512u : 1024u);
+    float n = (float)p.N;
+    for (uint32_t g = 1; g < p.ngroups && g < 3; g++) n += (float)p.Nx[g - 1];
+    const float mb = n * (float)p.col_bytes * 1e-6f, mk = (float)p.M * (float)p.K;
+    const uint32_t cw = gemv_tile_columns(p), ks = split ? skinny_ksplit(p) : gemm_base_ksplit(p);
+    auto per_cu = [](uint64_t wgs) { return (float)((wgs + 255) / 256); };
+    const FewCost& c = few_cost(f);
+    const float wgs = per_cu(column_tiles(p, cw));
+    const float few = price(cw == 32 ? c.few32 : c.few16, mb, wgs * (float)((p.K / 256 + 7) / 8), wgs * mk * 1e-5f, mk * 1e-5f);
+    const float steps = per_cu((uint64_t)column_tiles(p, split ? 64 : 128) * ks) * (float)p.K / (256.0f * (float)ks);
+    const float partials = (float)ks * (float)p.M * n * 1e-6f;
+    const float other = split ? price(c.split, mb, steps, partials, (float)ks)
+                              : price(c.tiles, mb, steps, ks > 1 ? 1.0f : 0.0f, partials);
+    return few < 0.94f * other;
 }
-
-// Two column tiles per workgroup when the workgroups of one would not be
-// resident at once (MLX N = 14336, K = 4096, M = 1: 15.5 -> 12.8 us).
-uint32_t gemv_tile_columns(const GemmParams& p) { return !p.W2 && column_tiles(p, 16) > 512 ? 32 : 16; }
 
 template <int F>
 static hipError_t launch_gemv_f(const GemmParams& p, hipStream_t st) {

@@ -303,6 +303,13 @@ def test_projection_plan_measured(lib, fmt, M, K, N, swiglu, want):
     (6, 11, 5632, 6144, False, True),     # 16.7 / 29.7
     (4, 4, 14336, 14336, True, True),     # 1.7x
     (1, 1, 4096, 14336, True, True),      # 21.3 / 33.2
+    # K that splits badly (42, 54, 30 super-blocks), and workgroups uneven over the CUs
+    (2, 16, 10752, 1416, False, True),    # 14.2 / 45.4
+    (3, 12, 13824, 3712, False, True),    # 15.8 / 37.9
+    (6, 14, 7680, 936, False, True),      # 11.4 / 26.6
+    (1, 7, 7168, 8720, False, False),     # 18.0 / 24.5
+    (1, 3, 6144, 9544, False, False),     # 16.2 / 21.1
+    (8, 4, 7680, 9056, False, False),     # 19.4 / 22.6
 ])
 def test_projection_plan_few_rows(lib, fmt, M, K, N, swiglu, few):
     got = m4_bridge.projection_plan(lib, fmt, M, K, N, swiglu=swiglu).kernel_name
