@@ -273,6 +273,7 @@ def test_projection_plan(lib):
     (6, 256, 2048, 4096, True, (128, 128, 1, 4)),     # 27.8 / 35.7 (no split)
     (0, 128, 2048, 8192, True, (128, 128, 1, 4)),     # 26.0 / 29.3
     (6, 504, 4096, 4096, True, (128, 128, 1, 2)),     # 57.8 / 71.9
+    (0, 5264, 1792, 3840, True, (256, 128, 1, 1)),    # MLP with the down projection 268 / 278 (128 x 128)
     # gains over the base plan that stay
     (1, 77, 8192, 2048, False, (64, 128, 1, 8)),      # 16.4 / 20.8 (128 x 128, 16 splits)
     (8, 8192, 4096, 14336, True, (256, 128, 1, 1)),   # 1660 / 1909 (128 x 128)
