@@ -252,10 +252,11 @@ __global__ void __launch_bounds__(256) kv_prep_kernel(const void* Ksrc, const vo
 // barrier ties them): 4 / NK blocks of 32 queries times NK key groups, group kg
 // taking the kg-th share of every tile's 32-key units, the partial states
 // merged through LDS at the end of a query tile.  Per 32 x 32 unit a wave issues
-// D / 16 MFMAs for S^T = K . Q^T, a softmax of ~85 VALU ops and 16 exponentials
-// (16 cycles each) and D / 16 MFMAs for O^T += V^T . P^T, and reads 128 D bytes
-// of LDS; at D = 128 the three take about the same time, at D = 64 the VALU is
-// what bounds it.
+// D / 16 MFMAs for S^T = K . Q^T, a softmax of ~90 VALU ops, 16 of them
+// exponentials (16 cycles each), and D / 16 MFMAs for O^T += V^T . P^T, and reads
+// 128 D bytes of LDS.  Counters: D = 128, M = 8100 5.6 VALU ops per MFMA (90 per unit),
+// the matrix pipe 50% busy at 1.8 GHz; D = 64, M = 2048 12.9 (103 per unit, masks and
+// merges included), 18% busy, waves waiting 37% of their cycles.
 //
 // Key tiles of 32 KB (K rows, then V^T rows) are double-buffered in LDS, copied
 // there by buffer loads in inline asm one tile ahead; the only barrier is one
@@ -267,10 +268,10 @@ __global__ void __launch_bounds__(256) kv_prep_kernel(const void* Ksrc, const vo
 //
 // Before, one 8-wave workgroup per CU (4 waves at D = 128, one per SIMD) ran an
 // in-wave software pipeline of the two phases; at one wave per SIMD the compiler
-// moved the accumulators between register files (168 VALU ops per unit instead
-// of ~85) and nothing covered its waits.  us with the cache pass, before ->
-// now: D = 128, H = 32, Hkv = 8, M = 8100 974 -> 582; M = 1000 49.4 -> 27.5;
-// D = 64, H = 32, M = 2048 42.5 -> 40.3, M = 8192 433 -> 370, M = 500 19.5 -> 12.5.
+// moved the accumulators between register files (11.7 VALU ops per MFMA at D = 128, M =
+// 2048) and nothing covered its waits.  us with the cache pass, before ->
+// now: D = 128, H = 32, Hkv = 8, M = 8100 984 -> 578; M = 1000 49.4 -> 27.5;
+// D = 64, H = 32, M = 2048 42.7 -> 39.9, M = 8192 433 -> 370, M = 500 19.5 -> 12.5.
 // --------------------------------------------------------------------------
 constexpr int tile_keys(int D) { return D == 64 ? 128 : 64; }  // 32 KB of K and V^T per tile at either width
 constexpr int kTileBytes = 32768;
@@ -446,7 +447,7 @@ __global__ void __launch_bounds__(256, 2) flash_attn_kernel(AttnParams p, int pa
             l_run *= alpha;
         }
         // raised wave priority over the exponentials and their MFMAs: the SIMD's
-        // other wave, in its S phase, yields (M = 8100, D = 128 596 -> 585 us)
+        // other wave, in its S phase, yields (M = 8100, D = 128 2% faster)
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int b = 0; b < NB; b++) {

@@ -26,7 +26,7 @@ enum QuantFormat : int {
     // scale and bias followed by its eight uint32 code words exactly as MLX
     // packs them (element 8j + i in bits 4i of word j).  Not in the
     // reference, whose MLX_4BIT block is 32 elements (quant_router.h:41-45);
-    // BASELINE's MLX configuration is this layout (4.5 bits per weight).
+    // MLX's own layout (4.5 bits per weight).
     QUANT_MLX_4BIT_G64 = 8,
     QUANT_CUSTOM = 99,
 };

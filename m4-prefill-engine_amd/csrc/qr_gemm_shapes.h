@@ -22,7 +22,7 @@ namespace qr {
 //                  of two column waves take alternate K steps and meet in LDS,
 //                  so 224 workgroups cover M = 128, N = 14336 with no K split)
 //   2 (SwiGLU): 4, 1, 4 -> 128 x 128 outputs (gate + up: 256 weight columns)
-//   7, 8 (SwiGLU): 256 x 256, 256 x 128 outputs (qr_gemm_wide.hip)
+//   7, 8 (SwiGLU): 256 x 256, 256 x 128 outputs (qr_gemm_wide.hip), never a base
 #define QR_RB_BIG 4, 2, 4, 1, 1
 #define QR_RB_BIG_K 4, 1, 8, 1, 1
 #define QR_RB_MID 4, 1, 4, 1, 1
@@ -42,13 +42,13 @@ constexpr bool wide_format(int f) {
 }
 // Formats whose 128 x 256 tiles are shape 3 (8 waves), not 0.
 constexpr bool big_k_format(int f) { return f == QUANT_Q4_K || f == QUANT_TERNARY_1_58; }
-// Base shape choice (gemm_plan compares it with the others by tile count).  At M >= 1024 the wide tile is used while it alone fills the
-// 256 CUs; when it cannot (N small), 128 x 128 tiles give twice the tiles, so
-// the K split -- whose fp32 partials are M x N x 4 bytes written and read per
+// Base shape choice (gemm_plan compares its price with the others').  At M >= 1024
+// the 128 x 256 tile is used while it alone fills the 256 CUs; when it cannot (N
+// small), 128 x 128 tiles give twice the tiles, so the K split -- whose fp32 partials are M x N x 4 bytes written and read per
 // extra split -- is halved or avoided.
 inline int rb_pick(int format, uint32_t M, uint32_t N, uint32_t K, bool dual) {
     if (dual) return 2;
-    // The 3/5-bit double-rounding formats (no BASELINE configuration) keep
+    // The 3/5-bit double-rounding formats keep
     // one tile shape: fewer instances of their heavy fp64 decode to compile.
     if (format == QUANT_VAR_RATE_AFFINE || format == QUANT_EXL3) return 1;
     // K groups instead of a K split: one 128-row tile, enough 64-column tiles
@@ -72,7 +72,7 @@ inline int rb_pick(int format, uint32_t M, uint32_t N, uint32_t K, bool dual) {
     if (cheap && tail != 0 && tail <= 64) {
         // the same tile as two K groups of four waves (two per SIMD, each
         // taking alternate steps: half the serial steps per wave) when the
-        // grid needs no K split anyway (cfg4: 15.6 -> 14.5 us)
+        // grid needs no K split anyway (ternary M = 129, K = 2048, N = 8192: 15.6 -> 14.5 us)
         if (K % 128 == 0 && ((M + 63) / 64) * ((N + 127) / 128) > 128) return 6;
         return 4;
     }

@@ -1,6 +1,6 @@
 // qr_gemm_skinny.hip -- weight-streaming projection for small M (M <= 64).
 //
-// The M=33 prefill projection is bound by streaming the
+// The M=33 prefill projection (Q4_0, K = N = 4096) is bound by streaming the
 // packed weights from HBM; the reference's 64x64 tiling (quant_router_kernels.
 // metal:442-581) leaves 31 of 64 rows idle and launches only N/64 groups.
 // Here every CU streams its own slice of W:

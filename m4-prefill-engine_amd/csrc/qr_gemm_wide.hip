@@ -21,9 +21,9 @@
 //  * Decode, copies and fragment reads are spread over four chunks per k-slice
 //    between the MFMAs.
 // Measured (MLX g64, M = 8192, K = 4096, N = 14336, SwiGLU and down projection)
-// 2725 -> 2359 us, i.e. 1.06 -> 1.22 PF; Q4_K at M = 1000, N = 14336 170.9 ->
-// 118.3 us.  The matrix pipe is ~67% busy at ~1.6 GHz; the same loop with
-// nothing but its MFMAs reaches 1.45 PF, where the clock is what limits.
+// 2762 -> 2365 us, i.e. 1.04 -> 1.22 PF; Q4_K SwiGLU at M = 1000, K = 4096, N = 14336
+// 309 -> 241 us.  The matrix pipe is 67% busy at 1.65 GHz (counters, g64), 2.0 - 2.2
+// VALU ops and 0.7 LDS ops per MFMA; 47% at 2.0 GHz for Q4_K at M = 1000 (3.1 VALU ops).
 #include "qr_decode.h"
 #include "qr_gemm_shapes.h"
 
@@ -51,8 +51,8 @@ struct Cfg {
 // 64-byte LDS rows hold a row's 32 k values as four 16-byte units; unit u of
 // row r sits at u ^ swz(r), chosen so that 16 lanes reading one unit hit distinct
 // banks both for 16 consecutive rows and for the rows {0-3, 12-15, 20-27} /
-// {4-11, 16-19, 28-31} (with a swizzle good for consecutive rows only, the
-// conflict counter read 3.0e7 instead of 5e5 cycles at M = 8192, N = 4096, K = 14336).
+// {4-11, 16-19, 28-31} (M = 8192, N = 4096, K = 14336: 5.2e5 conflict cycles in 2.0e7
+// LDS instructions).
 __device__ __forceinline__ uint32_t swz(uint32_t r) { return ((r >> 2) & 3u) ^ (r & 2u); }
 // 128-byte rows (X of a pair of steps): unit u of row r at u ^ xswz(r).
 __device__ __forceinline__ uint32_t xswz(uint32_t r) { return (r ^ (r >> 3)) & 7u; }
